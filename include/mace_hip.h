@@ -115,7 +115,10 @@ enum mh_kernel_kind {
     MH_EDGE_BWD = 76,    /* the harmonics' and the embedding's backward in one pass                      */
     MH_MLP_BWD_P = 77,   /* radial MLP backward over shared rows, an edge's and its partner's gW0 summed   */
     MH_LIN_BWD_SUM = 78, /* node linear backward over the sum of three gradients of its output               */
-    MH_NUM_KINDS = 79
+    MH_CONV_FWD_P = 79,  /* MH_CONV_FWD with four wave groups per receiver (few receivers)                     */
+    MH_CONV_FWD_CP = 80, /* MH_CONV_FWD_C likewise                                                             */
+    MH_CONV_FWD_CRP = 81,/* MH_CONV_FWD_CR likewise                                                            */
+    MH_NUM_KINDS = 82
 };
 
 /* flags of mh_conv_bwd */

@@ -37,6 +37,7 @@ struct Kernel {
     int block = 0;
     int rows_per_block = 1;
     int grid_y = 1;          // second grid dimension (a fixed count: output blocks of a node linear)
+    int64_t resident = 0;    // workgroups that fit on the device at once (kinds that choose by it; see bind_grid)
 };
 
 }  // namespace
@@ -66,8 +67,9 @@ int hip_fail(hipError_t e, const char* what) {
         if (e_ != hipSuccess) return hip_fail(e_, #call); \
     } while (0)
 
-// Launch `kind` over `rows` rows; args are the kernel's parameters in order.
-int launch(mh_module* m, int kind, int64_t rows, void** args, void* stream, const char* what) {
+// Launch `kind` over `rows` rows; args are the kernel's parameters in order.  `grid_y`: the second grid dimension,
+// where the call chooses it (0: the bound one).
+int launch(mh_module* m, int kind, int64_t rows, void** args, void* stream, const char* what, int grid_y = 0) {
     if (!m) return fail(-1, std::string(what) + ": null module");
     const Kernel& k = m->k[kind];
     if (!k.fn) return fail(-1, std::string(what) + ": kernel slot not bound in this module");
@@ -82,7 +84,8 @@ int launch(mh_module* m, int kind, int64_t rows, void** args, void* stream, cons
     }
     int64_t grid = (rows + k.rows_per_block - 1) / k.rows_per_block;
     if (grid > 0x7fffffffLL) return fail(-1, std::string(what) + ": launch too large");
-    hipError_t e = hipModuleLaunchKernel(k.fn, static_cast<unsigned>(grid), static_cast<unsigned>(k.grid_y), 1,
+    hipError_t e = hipModuleLaunchKernel(k.fn, static_cast<unsigned>(grid),
+                                         static_cast<unsigned>(grid_y > 0 ? grid_y : k.grid_y), 1,
                                          static_cast<unsigned>(k.block), 1, 1, 0, static_cast<hipStream_t>(stream), args,
                                          nullptr);
     if (e != hipSuccess) return hip_fail(e, what);
@@ -139,7 +142,7 @@ extern "C" {
 
 const char* mh_last_error(void) { return g_err.c_str(); }
 
-int mh_version(void) { return 42; }
+int mh_version(void) { return 43; }
 
 int mh_launch_log(int enable) {
     std::lock_guard<std::mutex> lock(g_log_mu);
@@ -252,6 +255,11 @@ int mh_module_bind_grid(mh_module* m, int kind, const char* name, int block_thre
     m->k[kind].block = block_threads;
     m->k[kind].rows_per_block = rows_per_block;
     m->k[kind].grid_y = grid_y;
+    if (kind == MH_CONV_FWD_P || kind == MH_CONV_FWD_CP || kind == MH_CONV_FWD_CRP) {
+        int fit = 0;
+        if (int rc = resident_blocks(m, kind, &fit)) return rc;
+        m->k[kind].resident = fit;
+    }
     return 0;
 }
 
@@ -259,10 +267,43 @@ int mh_module_bind(mh_module* m, int kind, const char* name, int block_threads, 
     return mh_module_bind_grid(m, kind, name, block_threads, rows_per_block, 1);
 }
 
+}  // extern "C"
+
+namespace {
+
+// The convolution forward's kernel for N receivers: `grouped` (four wave groups per receiver, each a quarter of its
+// edges) where it is bound and its workgroups do not fill the device more than 1.6 times over, else `plain`.  A
+// receiver's edges are one serial chain in the plain kernel, so few receivers leave the chip idle; many receivers fill
+// it and the grouped kernel's LDS sums only cost.  Measured (us, plain / grouped; resident workgroups 512 for the
+// 1280-weight layer, 256 for the 2176-weight one, 1,024 for the 512-weight one): 1280 weights N = 108 31.4 / 13.5, 400
+// 34.2 / 20.9, 720 41.8 / 36.8, 1176 53.4 / 58.2; 2176 weights N = 108 59.8 / 26.6, 400 65.4 / 53.0, 720 79.8 / 81.5;
+// 512 weights N = 108 11.9 / 8.7, 1176 31.9 / 24.0, 2048 36.9 / 40.3.
+int fwd_kind(const mh_module* m, int plain, int grouped, int64_t N) {
+    if (!m || !m->k[grouped].fn) return plain;
+    return 5 * N <= 8 * m->k[grouped].resident ? grouped : plain;
+}
+
+// Workgroups per receiver of the receiver-ordered backward (each takes a slice of the receiver's edges, whose outputs
+// are per edge; each loads the receiver's g row again).  By the waves that one workgroup per receiver would make,
+// against 1,024 SIMDs.  Measured (us, 1 / 2 / 4 / 8 per receiver): 1280 weights (two waves) N = 108 56.8 / 31.3 / 19.7
+// / 16.0, 400 63.0 / 43.5 / 47.4 / 40.6, 1176 120 / 117 / 115 / 114, 2048 215 / 191 / 192 / 198, 3600 339 / 321 / 326 /
+// 342, 7056 618 / 614 / 626 / 658; 2176 weights N = 1176 258 / 211 / 201 / 214, 3600 576 / 577 / 586 / 625; 512 weights
+// N = 108 28.1 / 16.2 / 11.1 / 8.5, 2048 79 / 70 / 70 / 77, 7056 283 / 297 / 286 / 297; 96 weights (one wave) N = 1176
+// 39.9 / 25.0 / 17.8 / 19.6, 7056 112 / 94 / 97 / 103.
+int bwd_parts(const mh_module* m, int kind, int64_t N) {
+    if (!m) return 1;
+    const int64_t waves = N * (m->k[kind].block / 64);
+    return waves <= 384 ? 8 : waves <= 3072 ? 4 : waves <= 8192 ? 2 : 1;
+}
+
+}  // namespace
+
+extern "C" {
+
 int mh_conv_fwd(mh_module* m, const float* x, const float* Y, const float* W, const int32_t* rowptr,
                 const int32_t* eids, const int32_t* senders, float* out, int32_t N, void* stream) {
     void* args[] = {&x, &Y, &W, &rowptr, &eids, &senders, &out, &N};
-    return launch(m, MH_CONV_FWD, N, args, stream, "mh_conv_fwd");
+    return launch(m, fwd_kind(m, MH_CONV_FWD, MH_CONV_FWD_P, N), N, args, stream, "mh_conv_fwd");
 }
 
 int mh_conv_fwd_cut_rows(mh_module* m, const float* x, const float* Y, const float* W, const int32_t* rowptr,
@@ -271,7 +312,8 @@ int mh_conv_fwd_cut_rows(mh_module* m, const float* x, const float* Y, const flo
     if (!cutoff) return fail(-1, "mh_conv_fwd_cut: cutoff is NULL");
     void* args[] = {&x, &Y, &W, &rowptr, &eids, &senders, &out, &N, &cutoff, &wrow};
     // a row map: the kernel variant whose W0 loads are cacheable (shared rows are read twice)
-    return launch(m, wrow ? MH_CONV_FWD_CR : MH_CONV_FWD_C, N, args, stream, "mh_conv_fwd_cut");
+    return launch(m, wrow ? fwd_kind(m, MH_CONV_FWD_CR, MH_CONV_FWD_CRP, N) : fwd_kind(m, MH_CONV_FWD_C, MH_CONV_FWD_CP, N),
+                  N, args, stream, "mh_conv_fwd_cut");
 }
 
 int mh_conv_fwd_cut(mh_module* m, const float* x, const float* Y, const float* W, const int32_t* rowptr,
@@ -311,10 +353,11 @@ int mh_conv_bwd_recv_rows(mh_module* m, const float* x, const float* g, const fl
     if (cutoff) {
         void* args[] = {&x, &g, &Y, &W, &rowptr_r, &eids_r, &senders, &gW, &gY, &work, &N, &kflags, &cutoff,
                         &g_cutoff, &wrow};
-        rc = launch(m, MH_CONV_BWD_RC, N, args, stream, "mh_conv_bwd_recv (factored weights)");
+        rc = launch(m, MH_CONV_BWD_RC, N, args, stream, "mh_conv_bwd_recv (factored weights)",
+                    bwd_parts(m, MH_CONV_BWD_RC, N));
     } else {
         void* args[] = {&x, &g, &Y, &W, &rowptr_r, &eids_r, &senders, &gW, &gY, &work, &N, &kflags};
-        rc = launch(m, MH_CONV_BWD_R, N, args, stream, "mh_conv_bwd_recv");
+        rc = launch(m, MH_CONV_BWD_R, N, args, stream, "mh_conv_bwd_recv", bwd_parts(m, MH_CONV_BWD_R, N));
     }
     if (rc || !want_gx) return rc;
     const float* msg = work;

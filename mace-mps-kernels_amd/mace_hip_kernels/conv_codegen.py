@@ -80,6 +80,14 @@ GY_LDS_ATOMIC = True
 CHUNK_LDS = 24576
 
 
+# Forward with few receivers: FWD_GROUPS wave groups of one workgroup share a receiver, each walking its own slice of
+# the receiver's edges (chunks of GROUP_CHUNK edges), and their partial sums are added in LDS in a fixed order
+# (conv_fwd*p_*).  A receiver's edges are one serial chain of about 1 us each, so with fewer workgroups than the chip
+# holds the chain is the kernel's time; FWD_GROUPS slices cut it to a quarter.
+FWD_GROUPS = 4
+GROUP_CHUNK = 16
+
+
 class _Gen:
     """Shared naming and code fragments for the kernels of one spec."""
 
@@ -102,8 +110,10 @@ class _Gen:
         self.np = len(self.pairs)
         self.npp = (self.np + 3) // 4 * 4
 
-    def prelude(self):
-        L = ['  const int u = threadIdx.x, lane = threadIdx.x & (MH_WAVE - 1), wave = threadIdx.x >> 6;']
+    def prelude(self, groups=1):
+        L = ['  const int u = threadIdx.x, lane = threadIdx.x & (MH_WAVE - 1), wave = threadIdx.x >> 6;'] if groups == 1 else [
+            '  const int grp = __builtin_amdgcn_readfirstlane(threadIdx.x / BLOCK);      // wave group (wave-uniform)',
+            '  const int u = threadIdx.x - grp * BLOCK, lane = threadIdx.x & (MH_WAVE - 1), wave = u >> 6;']
         if self.full:
             L += ['  const bool active = true;', '  const unsigned uc = u;']
         else:
@@ -279,6 +289,15 @@ def chunk_edges(npp):
     return WAVE if WAVE * npp * 4 <= CHUNK_LDS else WAVE // 2
 
 
+def fwd_groups(spec):
+    """Wave groups per receiver of the forward's few-receivers kernels, 0 where they do not fit: a workgroup has at
+    most 1024 threads, and its partial sums and coupling products must fit a compute unit's LDS."""
+    no = sum(co['d3'] for co in spec.coef)
+    npp = (len({(co['k'], a, c) for co in spec.coef for a, _, c, _ in co['terms']}) + 3) // 4 * 4
+    lds = 4 * (FWD_GROUPS // 2 * no * spec.block + FWD_GROUPS * GROUP_CHUNK * (npp + spec.ncb))
+    return FWD_GROUPS if FWD_GROUPS * spec.block <= 1024 and lds <= 153600 else 0
+
+
 def _gy_combine(indent, edge_expr, cut=False, atomic=False):
     """Sum the per-wave gY partials of the current chunk held in LDS and write gY rows (fixed order); with ``cut``
     also the ∂/∂c partials.  The leading barrier also orders the chunk's Ms reads before the next chunk's prologue
@@ -329,54 +348,81 @@ def source(spec):
     ms_decl_c = ['  __shared__ float4 Ms4[CHUNK][NPP / 4];',
                  '  float (*Ms)[NPP] = reinterpret_cast<float (*)[NPP]>(Ms4);']
     # ------------------------------------------------------------------------------------------- forward
-    def fwd_kernel(cut, rows=False):
+    def fwd_kernel(cut, rows=False, groups=1):
         """``cut`` (kernel ``conv_fwdc``): the weights are W0·c with a per-edge scalar c, read as W0 and scaled in
         registers (the product is never formed in memory); an edge with c == 0 (padding, or past r_max in a
         neighbour list with a skin) contributes exactly zero, so each chunk of 64 edges is first compacted to its
         edges with c != 0 (ballot, then a per-wave LDS scatter by lane rank) and only those are walked.  Every wave
-        of the workgroup builds the same list, so the barriers stay uniform."""
+        of the workgroup builds the same list, so the barriers stay uniform.
+
+        ``groups`` > 1 (kernels ``conv_fwd*p``): that many wave groups per receiver, group i walking the i-th slice of
+        its edges in chunks of GROUP_CHUNK; the chunk count is the longest slice's, so that every wave meets every
+        barrier, and the groups' accumulators are added pairwise in LDS (i + i + half, half = groups / 2, ..., 1)."""
+        G2 = groups > 1
+        base = ("conv_fwdcr" if rows else "conv_fwdc") if cut else "conv_fwd"
+        pf = 1 if G2 else FWD_PREFETCH
+        ms = 'Ms4s[grp]' if G2 else 'Ms4'
         F = [
-            f'extern "C" __global__ __launch_bounds__(BLOCK) void '
-            f'{spec.kname(("conv_fwdcr" if rows else "conv_fwdc") if cut else "conv_fwd")}(',
+            f'extern "C" __global__ __launch_bounds__({f"{groups} * BLOCK" if G2 else "BLOCK"}) void '
+            f'{spec.kname(base + ("p" if G2 else ""))}(',
             '    const float* __restrict__ x, const float* __restrict__ Y, const float* __restrict__ W,',
             '    const int* __restrict__ rowptr, const int* __restrict__ eids, const int* __restrict__ senders,',
             '    float* __restrict__ out, int N' + (', const float* __restrict__ cutv, const int* __restrict__ wrow) {'
                                                    if cut else ') {'),
-        ] + ms_decl_c + (['  __shared__ int sidx[NCB][CHUNK];'] if cut else []) + [
+        ]
+        if G2:
+            F += [f'  __shared__ float4 Ms4s[{groups}][{GROUP_CHUNK}][NPP / 4];',
+                  f'  __shared__ float red[{groups // 2}][{no}][BLOCK];']
+            F += [f'  __shared__ int sidxs[{groups}][NCB][{GROUP_CHUNK}];'] if cut else []
+        else:
+            F += ms_decl_c + (['  __shared__ int sidx[NCB][CHUNK];'] if cut else [])
+        F += [
             '  const int n = mh_xcd_block(blockIdx.x, gridDim.x);',
             '  if (n >= N) return;',
-        ] + G.prelude() + [
+        ] + G.prelude(groups)
+        if G2:
+            F += [f'  float4 (*Ms4)[NPP / 4] = {ms};',
+                  '  float (*Ms)[NPP] = reinterpret_cast<float (*)[NPP]>(Ms4);']
+            F += [f'  int (*sidx)[{GROUP_CHUNK}] = sidxs[grp];'] if cut else []
+        F += [
             '  ' + decl('acc', no, '0.0f'),
             '  ' + decl('xn', nx), '  ' + decl('wn', nk),
-        ] + (['  ' + decl('xm', nx), '  ' + decl('wm', nk)] if FWD_PREFETCH > 1 else []) + [
-            '  const int p0 = rowptr[n], p1 = rowptr[n + 1];',
-            '  for (int pb = p0; pb < p1; pb += CHUNK) {',
-        ]
+        ] + (['  ' + decl('xm', nx), '  ' + decl('wm', nk)] if pf > 1 else [])
+        if G2:
+            F += ['  const int q0 = rowptr[n], q1 = rowptr[n + 1];',
+                  f'  const int per = (q1 - q0 + {groups - 1}) / {groups};      // edges of a slice (the last may be shorter)',
+                  '  const int p0 = min(q0 + grp * per, q1), p1 = min(p0 + per, q1);',
+                  f'  for (int c0 = 0; c0 < per; c0 += {GROUP_CHUNK}) {{',
+                  '    const int pb = p0 + c0;',
+                  f'    const int cnt0 = max(0, min({GROUP_CHUNK}, p1 - pb));']
+        else:
+            F += ['  const int p0 = rowptr[n], p1 = rowptr[n + 1];',
+                  '  for (int pb = p0; pb < p1; pb += CHUNK) {',
+                  '    const int cnt0 = min(CHUNK, p1 - pb);']
         if cut:
-            F += ['    const int cnt0 = min(CHUNK, p1 - pb);',
-                  '    int my_e = 0, my_s = 0;',
+            F += ['    int my_e = 0, my_s = 0;',
                   '    bool keep = false;',
                   '    if (lane < cnt0) { my_e = eids[pb + lane]; keep = cutv[my_e] != 0.0f; }',
                   '    const unsigned long long kept = __ballot(keep);',
                   '    const int cnt = __popcll(kept);',
-                  '    if (keep) sidx[wave][__popcll(kept & ((1ull << lane) - 1ull))] = my_e;',
-                  '    if (cnt == 0) continue;',
-                  '    float my_c = 0.0f;',
+                  '    if (keep) sidx[wave][__popcll(kept & ((1ull << lane) - 1ull))] = my_e;']
+            F += [] if G2 else ['    if (cnt == 0) continue;']
+            F += ['    float my_c = 0.0f;',
                   '    int my_w = 0;                       // the W0 row of lane j\'s edge (its own, or wrow[e])',
                   '    if (lane < cnt) {',
                   '      my_e = sidx[wave][lane]; my_s = senders[my_e]; my_c = cutv[my_e];',
                   '      my_w = wrow ? wrow[my_e] : my_e;',
                   '    }']
         else:
-            F += ['    const int cnt = min(CHUNK, p1 - pb);',
+            F += ['    const int cnt = cnt0;',
                   '    int my_e = 0, my_s = 0;',
                   '    if (lane < cnt) { my_e = eids[pb + lane]; my_s = senders[my_e]; }',
                   '    const int my_w = my_e;']
         F += G.m_prologue('    ', 'my_e')
-        F += ['    {', '      const int er0 = mh_bcast(my_w, 0), s0 = mh_bcast(my_s, 0);']
+        F += ['    if (cnt > 0) {' if G2 else '    {', '      const int er0 = mh_bcast(my_w, 0), s0 = mh_bcast(my_s, 0);']
         F += G.ld_x('      ', 's0', 'xn') + G.ld_w('      ', 'er0', 'wn', W_NT_ROWS if rows else W_NT)
         F += ['    }']
-        if FWD_PREFETCH > 1:          # edge 1 (or the last edge again) one stage further out
+        if pf > 1:          # edge 1 (or the last edge again) one stage further out
             F += ['    {', '      const int er1 = mh_bcast(my_w, min(1, cnt - 1)), s1 = mh_bcast(my_s, min(1, cnt - 1));']
             F += G.ld_x('      ', 's1', 'xm') + G.ld_w('      ', 'er1', 'wm', W_NT_ROWS if rows else W_NT)
             F += ['    }']
@@ -387,7 +433,7 @@ def source(spec):
             F += [f'      const float w{k} = wn{k} * cj;' for k in range(nk)]
         else:
             F += copy('w', 'wn', nk)
-        if FWD_PREFETCH > 1:
+        if pf > 1:
             # unconditional (the last edges re-load themselves): no branch around the loads
             F += [f'      xn{i} = xm{i};' for i in range(nx)] + [f'      wn{k} = wm{k};' for k in range(nk)]
             F += ['      {', '        const int j2 = min(j + 2, cnt - 1);',
@@ -399,13 +445,25 @@ def source(spec):
             F += G.ld_x('        ', 's1', 'xn') + G.ld_w('        ', 'er1', 'wn', W_NT_ROWS if rows else W_NT)
             F += ['      }']
         F += G.fwd_body('      ')
-        F += ['    }', '    __syncthreads();', '  }', '  if (active) {',
+        F += ['    }', '    __syncthreads();', '  }']
+        half = groups // 2
+        while half >= 1:
+            F += [f'  if (grp >= {half} && grp < {2 * half}) {{']
+            F += [f'    red[grp - {half}][{i}][u] = acc{i};' for i in range(no)]
+            F += ['  }', '  __syncthreads();', f'  if (grp < {half}) {{']
+            F += [f'    acc{i} += red[grp][{i}][u];' for i in range(no)]
+            F += ['  }'] + (['  __syncthreads();'] if half > 1 else [])
+            half //= 2
+        F += ['  if (grp == 0 && active) {' if G2 else '  if (active) {',
               '    float* __restrict__ o = out + (size_t)n * OUT_DIM;']
         for co in spec.coef:
             F += [f'    mh_st(o + {co["o3"] + c}, ol{co["d3"]}, acc{G.oi[co["k"]] + c});' for c in range(co['d3'])]
         return F + ['  }', '}', '']
 
     L += fwd_kernel(False) + fwd_kernel(True) + fwd_kernel(True, rows=True)
+    if fwd_groups(spec):
+        for kw in (dict(cut=False), dict(cut=True), dict(cut=True, rows=True)):
+            L += fwd_kernel(**kw, groups=FWD_GROUPS)
     # ----------------------------------------------------------------------------------- fused backward
     L += [
         f'extern "C" __global__ __launch_bounds__(BLOCK) void {spec.kname("conv_bwd")}(',
@@ -531,6 +589,11 @@ def _bwd_recv(G, gyr, pdecl, decl, copy, cut=False):
         '  float (*Ms)[NPP] = reinterpret_cast<float (*)[NPP]>(Ms4);',
         '  const int r = mh_xcd_block(blockIdx.x, gridDim.x);',
         '  if (r >= N) return;',
+        '  // this workgroup\'s slice of the receiver\'s edges (gridDim.y of them; every output is per edge)',
+        '  const int q0 = rowptr[r], q1 = rowptr[r + 1];',
+        '  const int per = (q1 - q0 + (int)gridDim.y - 1) / (int)gridDim.y;',
+        '  const int p0 = min(q0 + (int)blockIdx.y * per, q1), p1 = min(p0 + per, q1);',
+        '  if (p0 >= p1) return;',
     ] + ([
         '  for (int q = threadIdx.x; q < CHUNK * Y_PAD; q += BLOCK) (&part[0][0])[q] = 0.0f;',
     ] + (['  for (int q = threadIdx.x; q < CHUNK; q += BLOCK) partc[q] = 0.0f;'] if cut else []) + [
@@ -545,7 +608,6 @@ def _bwd_recv(G, gyr, pdecl, decl, copy, cut=False):
     L += ['  ' + decl('xn', nx), '  ' + decl('wn', nk)]
     if BWD_PREFETCH > 1:
         L += ['  ' + decl('xm', nx), '  ' + decl('wm', nk)]
-    L += ['  const int p0 = rowptr[r], p1 = rowptr[r + 1];']
 
     def chunks(msg):
         C = ['  for (int pb = p0; pb < p1; pb += CHUNK) {']
