@@ -115,10 +115,7 @@ enum mh_kernel_kind {
     MH_EDGE_BWD = 76,    /* the harmonics' and the embedding's backward in one pass                      */
     MH_MLP_BWD_P = 77,   /* radial MLP backward over shared rows, an edge's and its partner's gW0 summed   */
     MH_LIN_BWD_SUM = 78, /* node linear backward over the sum of three gradients of its output               */
-    MH_CONV_FWD_P = 79,  /* MH_CONV_FWD with four wave groups per receiver (few receivers)                     */
-    MH_CONV_FWD_CP = 80, /* MH_CONV_FWD_C likewise                                                             */
-    MH_CONV_FWD_CRP = 81,/* MH_CONV_FWD_CR likewise                                                            */
-    MH_NUM_KINDS = 82
+    MH_NUM_KINDS = 79
 };
 
 /* flags of mh_conv_bwd */
@@ -167,6 +164,10 @@ int mh_module_bind(mh_module* m, int kind, const char* name, int block_threads, 
 /* As mh_module_bind, with a second grid dimension of grid_y workgroups (1..65535); mh_module_bind uses 1. */
 int mh_module_bind_grid(mh_module* m, int kind, const char* name, int block_threads, int rows_per_block,
                         int grid_y);
+/* The kernel bound to `kind` may also be launched with groups x block_threads threads and lds_bytes of dynamic LDS
+ * (the convolution forwards: conv_codegen.fwd_groups and fwd_groups_lds give both), in which `groups` wave groups
+ * share each row; the entry points choose that form for small launches.  Without this call they never do. */
+int mh_module_bind_groups(mh_module* m, int kind, int groups, int lds_bytes);
 
 /* Fused convolution forward: out[n] = Σ_{p in rowptr[n]..rowptr[n+1]} TP(x[senders[e]], Y[e], W[e]), e = eids[p].
  * rowptr/eids: receiver-sorted CSR.  Replaces lib.conv_fwd (reference conv.py:109-141, launched at conv.py:247). */

@@ -37,7 +37,9 @@ struct Kernel {
     int block = 0;
     int rows_per_block = 1;
     int grid_y = 1;          // second grid dimension (a fixed count: output blocks of a node linear)
-    int64_t resident = 0;    // workgroups that fit on the device at once (kinds that choose by it; see bind_grid)
+    int groups = 1;          // the kernel also runs with groups x block threads and `lds` bytes of dynamic LDS
+    int lds = 0;             // (mh_module_bind_groups), of which `resident` workgroups fit on the device at once
+    int64_t resident = 0;
 };
 
 }  // namespace
@@ -68,8 +70,9 @@ int hip_fail(hipError_t e, const char* what) {
     } while (0)
 
 // Launch `kind` over `rows` rows; args are the kernel's parameters in order.  `grid_y`: the second grid dimension,
-// where the call chooses it (0: the bound one).
-int launch(mh_module* m, int kind, int64_t rows, void** args, void* stream, const char* what, int grid_y = 0) {
+// where the call chooses it (0: the bound one); `grouped`: the kernel's form of mh_module_bind_groups.
+int launch(mh_module* m, int kind, int64_t rows, void** args, void* stream, const char* what, int grid_y = 0,
+           bool grouped = false) {
     if (!m) return fail(-1, std::string(what) + ": null module");
     const Kernel& k = m->k[kind];
     if (!k.fn) return fail(-1, std::string(what) + ": kernel slot not bound in this module");
@@ -86,8 +89,9 @@ int launch(mh_module* m, int kind, int64_t rows, void** args, void* stream, cons
     if (grid > 0x7fffffffLL) return fail(-1, std::string(what) + ": launch too large");
     hipError_t e = hipModuleLaunchKernel(k.fn, static_cast<unsigned>(grid),
                                          static_cast<unsigned>(grid_y > 0 ? grid_y : k.grid_y), 1,
-                                         static_cast<unsigned>(k.block), 1, 1, 0, static_cast<hipStream_t>(stream), args,
-                                         nullptr);
+                                         static_cast<unsigned>(grouped ? k.groups * k.block : k.block), 1, 1,
+                                         static_cast<unsigned>(grouped ? k.lds : 0), static_cast<hipStream_t>(stream),
+                                         args, nullptr);
     if (e != hipSuccess) return hip_fail(e, what);
     {
         std::lock_guard<std::mutex> lock(g_log_mu);
@@ -255,11 +259,26 @@ int mh_module_bind_grid(mh_module* m, int kind, const char* name, int block_thre
     m->k[kind].block = block_threads;
     m->k[kind].rows_per_block = rows_per_block;
     m->k[kind].grid_y = grid_y;
-    if (kind == MH_CONV_FWD_P || kind == MH_CONV_FWD_CP || kind == MH_CONV_FWD_CRP) {
-        int fit = 0;
-        if (int rc = resident_blocks(m, kind, &fit)) return rc;
-        m->k[kind].resident = fit;
-    }
+    m->k[kind].groups = 1;
+    return 0;
+}
+
+int mh_module_bind_groups(mh_module* m, int kind, int groups, int lds_bytes) {
+    if (!m) return fail(-1, "mh_module_bind_groups: null argument");
+    if (kind < 0 || kind >= MH_NUM_KINDS || !m->k[kind].fn) return fail(-1, "mh_module_bind_groups: kind not bound");
+    Kernel& k = m->k[kind];
+    if (groups < 2 || groups * k.block > 1024 || lds_bytes < 0)
+        return fail(-1, "mh_module_bind_groups: bad launch shape");
+    MH_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k.fn), hipFuncAttributeMaxDynamicSharedMemorySize,
+                               lds_bytes));
+    int per_cu = 0, cus = 0;
+    MH_HIP(hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k.fn, groups * k.block,
+                                                              static_cast<size_t>(lds_bytes)));
+    MH_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, m->device));
+    if (per_cu < 1) return fail(-1, "mh_module_bind_groups: the grouped workgroup does not fit");
+    k.groups = groups;
+    k.lds = lds_bytes;
+    k.resident = static_cast<int64_t>(per_cu) * cus;
     return 0;
 }
 
@@ -271,16 +290,15 @@ int mh_module_bind(mh_module* m, int kind, const char* name, int block_threads, 
 
 namespace {
 
-// The convolution forward's kernel for N receivers: `grouped` (four wave groups per receiver, each a quarter of its
-// edges) where it is bound and its workgroups do not fill the device more than 1.6 times over, else `plain`.  A
-// receiver's edges are one serial chain in the plain kernel, so few receivers leave the chip idle; many receivers fill
-// it and the grouped kernel's LDS sums only cost.  Measured (us, plain / grouped; resident workgroups 512 for the
+// Whether the convolution forward over N receivers runs in its grouped form (four wave groups per receiver, each a
+// quarter of its edges): where that is bound and its workgroups do not fill the device more than 1.6 times over.  A
+// receiver's edges are one serial chain in the plain form, so few receivers leave the chip idle; many receivers fill
+// it and the grouped form's LDS sums only cost.  Measured (us, plain / grouped; resident workgroups 512 for the
 // 1280-weight layer, 256 for the 2176-weight one, 1,024 for the 512-weight one): 1280 weights N = 108 31.4 / 13.5, 400
 // 34.2 / 20.9, 720 41.8 / 36.8, 1176 53.4 / 58.2; 2176 weights N = 108 59.8 / 26.6, 400 65.4 / 53.0, 720 79.8 / 81.5;
 // 512 weights N = 108 11.9 / 8.7, 1176 31.9 / 24.0, 2048 36.9 / 40.3.
-int fwd_kind(const mh_module* m, int plain, int grouped, int64_t N) {
-    if (!m || !m->k[grouped].fn) return plain;
-    return 5 * N <= 8 * m->k[grouped].resident ? grouped : plain;
+bool fwd_grouped(const mh_module* m, int kind, int64_t N) {
+    return m && m->k[kind].groups > 1 && 5 * N <= 8 * m->k[kind].resident;
 }
 
 // Workgroups per receiver of the receiver-ordered backward (each takes a slice of the receiver's edges, whose outputs
@@ -303,7 +321,7 @@ extern "C" {
 int mh_conv_fwd(mh_module* m, const float* x, const float* Y, const float* W, const int32_t* rowptr,
                 const int32_t* eids, const int32_t* senders, float* out, int32_t N, void* stream) {
     void* args[] = {&x, &Y, &W, &rowptr, &eids, &senders, &out, &N};
-    return launch(m, fwd_kind(m, MH_CONV_FWD, MH_CONV_FWD_P, N), N, args, stream, "mh_conv_fwd");
+    return launch(m, MH_CONV_FWD, N, args, stream, "mh_conv_fwd", 0, fwd_grouped(m, MH_CONV_FWD, N));
 }
 
 int mh_conv_fwd_cut_rows(mh_module* m, const float* x, const float* Y, const float* W, const int32_t* rowptr,
@@ -312,8 +330,8 @@ int mh_conv_fwd_cut_rows(mh_module* m, const float* x, const float* Y, const flo
     if (!cutoff) return fail(-1, "mh_conv_fwd_cut: cutoff is NULL");
     void* args[] = {&x, &Y, &W, &rowptr, &eids, &senders, &out, &N, &cutoff, &wrow};
     // a row map: the kernel variant whose W0 loads are cacheable (shared rows are read twice)
-    return launch(m, wrow ? fwd_kind(m, MH_CONV_FWD_CR, MH_CONV_FWD_CRP, N) : fwd_kind(m, MH_CONV_FWD_C, MH_CONV_FWD_CP, N),
-                  N, args, stream, "mh_conv_fwd_cut");
+    const int kind = wrow ? MH_CONV_FWD_CR : MH_CONV_FWD_C;
+    return launch(m, kind, N, args, stream, "mh_conv_fwd_cut", 0, fwd_grouped(m, kind, N));
 }
 
 int mh_conv_fwd_cut(mh_module* m, const float* x, const float* Y, const float* W, const int32_t* rowptr,

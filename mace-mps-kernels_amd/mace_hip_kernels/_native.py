@@ -27,7 +27,7 @@ MH_CONV_FWD, MH_CONV_BWD, MH_CONV_BWD_WY, MH_SC_FWD, MH_SC_BWD, MH_CONV_BWD_R, M
     MH_SC_BWD_SI, MH_NL_SETUP, MH_NL_ZERO, MH_NL_BINS, MH_NL_SCAN, MH_NL_PLACE, MH_NL_COUNT, MH_NL_OFFSETS, \
     MH_NL_FILL, MH_SPECIES_ORDER, MH_MLP_JVP, MH_MLP_BWD2, MH_GEOM_SEGSUM, MH_NL_BASES, MH_EDGE_COUNT, \
     MH_EDGE_PLACE, MH_GEOM_SEGSUM1, MH_EDGE_PAIR, MH_CONV_FWD_CR, MH_MLP_H3, MH_MLP_OUT, MH_EDGE_FWD, \
-    MH_EDGE_BWD, MH_MLP_BWD_P, MH_LIN_BWD_SUM, MH_CONV_FWD_P, MH_CONV_FWD_CP, MH_CONV_FWD_CRP = range(82)
+    MH_EDGE_BWD, MH_MLP_BWD_P, MH_LIN_BWD_SUM = range(79)
 MH_WANT_GX, MH_WANT_GWY, MH_CUT_MASKED, MH_CUT_NOZERO = 1, 2, 4, 8
 ABI_VERSION = 43
 
@@ -50,6 +50,7 @@ _SIGS = {
     'mh_module_load': (ctypes.c_int, [_P, ctypes.c_size_t, ctypes.POINTER(_P)]),
     'mh_module_unload': (ctypes.c_int, [_P]),
     'mh_module_bind': (ctypes.c_int, [_P, ctypes.c_int, ctypes.c_char_p, ctypes.c_int, ctypes.c_int]),
+    'mh_module_bind_groups': (ctypes.c_int, [_P, ctypes.c_int, ctypes.c_int, ctypes.c_int]),
     'mh_conv_fwd': (ctypes.c_int, [_P] * 8 + [_I, _P]),
     'mh_conv_bwd_x': (ctypes.c_int, [_P] * 8 + [_I, _P]),
     'mh_conv_bwd_wy': (ctypes.c_int, [_P] * 9 + [_I, _P]),
@@ -202,6 +203,11 @@ class Module:
         for kind, (name, block, rows, *grid_y) in kernels.items():
             check(lib.mh_module_bind_grid(self.handle, kind, name.encode(), block, rows, grid_y[0] if grid_y else 1),
                   f'bind {name}')
+
+    def bind_groups(self, kinds, groups, lds):
+        """Let the kernels bound to ``kinds`` also run as ``groups`` wave groups per row (``mh_module_bind_groups``)."""
+        for kind in kinds:
+            check(self._lib.mh_module_bind_groups(self.handle, kind, groups, lds), 'bind groups')
 
     def __del__(self):
         h = getattr(self, 'handle', None)

@@ -30,7 +30,7 @@ import torch
 
 from . import _native, neighbours
 from .pending import stash_owner
-from .conv_codegen import fwd_groups, gxsum_block, source
+from .conv_codegen import fwd_groups, fwd_groups_lds, gxsum_block, source
 
 WAVE = 64
 
@@ -1017,13 +1017,8 @@ class HipConvTP(torch.nn.Module):
         self.source = source(self.spec)
         code = _native.compile_source(self.source)
         dev = torch.device(device) if device is not None else torch.device('cuda', torch.cuda.current_device())
-        groups = fwd_groups(self.spec)
-        grouped = {kind: (self.spec.kname(name), groups * self.spec.block, 1) for kind, name in (
-            (_native.MH_CONV_FWD_P, 'conv_fwdp'), (_native.MH_CONV_FWD_CP, 'conv_fwdcp'),
-            (_native.MH_CONV_FWD_CRP, 'conv_fwdcrp'))} if groups else {}
         with torch.cuda.device(dev):
             self.module = _native.Module(code, {
-                **grouped,
                 _native.MH_CONV_FWD: (self.spec.kname('conv_fwd'), self.spec.block, 1),
                 _native.MH_CONV_BWD: (self.spec.kname('conv_bwd'), self.spec.block, 1),
                 _native.MH_CONV_BWD_WY: (self.spec.kname('conv_bwd_wy'), self.spec.block, WAVE),
@@ -1033,6 +1028,10 @@ class HipConvTP(torch.nn.Module):
                 _native.MH_CONV_FWD_CR: (self.spec.kname('conv_fwdcr'), self.spec.block, 1),
                 _native.MH_CONV_GXSUM: (self.spec.kname('conv_gxsum'), gxsum_block(self.spec), 1),
             })
+            groups = fwd_groups(self.spec)
+            if groups:
+                self.module.bind_groups((_native.MH_CONV_FWD, _native.MH_CONV_FWD_C, _native.MH_CONV_FWD_CR), groups,
+                                        fwd_groups_lds(self.spec))
         self.irreps_in1, self.irreps_in2, self.irreps_out = tp.irreps_in1, tp.irreps_in2, tp.irreps_out
         self.instructions = tp.instructions
         self.weight_numel = tp.weight_numel

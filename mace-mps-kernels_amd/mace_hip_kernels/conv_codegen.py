@@ -80,12 +80,11 @@ GY_LDS_ATOMIC = True
 CHUNK_LDS = 24576
 
 
-# Forward with few receivers: FWD_GROUPS wave groups of one workgroup share a receiver, each walking its own slice of
-# the receiver's edges (chunks of GROUP_CHUNK edges), and their partial sums are added in LDS in a fixed order
-# (conv_fwd*p_*).  A receiver's edges are one serial chain of about 1 us each, so with fewer workgroups than the chip
-# holds the chain is the kernel's time; FWD_GROUPS slices cut it to a quarter.
+# Forward with few receivers: launched with FWD_GROUPS x BLOCK threads, FWD_GROUPS wave groups share a receiver, each
+# walking its own slice of the receiver's edges (in chunks of CHUNK / FWD_GROUPS), and their partial sums are added in
+# LDS in a fixed order.  A receiver's edges are one serial chain of about 1 us each, so with fewer workgroups than the
+# chip holds the chain is the kernel's time; FWD_GROUPS slices cut it to a quarter.
 FWD_GROUPS = 4
-GROUP_CHUNK = 16
 
 
 class _Gen:
@@ -290,12 +289,17 @@ def chunk_edges(npp):
 
 
 def fwd_groups(spec):
-    """Wave groups per receiver of the forward's few-receivers kernels, 0 where they do not fit: a workgroup has at
-    most 1024 threads, and its partial sums and coupling products must fit a compute unit's LDS."""
-    no = sum(co['d3'] for co in spec.coef)
+    """Wave groups per receiver of the forward kernels' few-receivers form, 0 where it does not fit: 512 threads (so
+    that the larger launch leaves the registers of the smaller one alone), and the partial sums beside the coupling
+    products within a compute unit's LDS."""
     npp = (len({(co['k'], a, c) for co in spec.coef for a, _, c, _ in co['terms']}) + 3) // 4 * 4
-    lds = 4 * (FWD_GROUPS // 2 * no * spec.block + FWD_GROUPS * GROUP_CHUNK * (npp + spec.ncb))
-    return FWD_GROUPS if FWD_GROUPS * spec.block <= 1024 and lds <= 153600 else 0
+    lds = fwd_groups_lds(spec) + 4 * chunk_edges(npp) * (npp + spec.ncb)
+    return FWD_GROUPS if FWD_GROUPS * spec.block <= 512 and lds <= 153600 else 0
+
+
+def fwd_groups_lds(spec):
+    """Dynamic LDS (bytes) of a forward launch with FWD_GROUPS wave groups: the accumulators of half of them."""
+    return 4 * (FWD_GROUPS // 2) * sum(co['d3'] for co in spec.coef) * spec.block
 
 
 def _gy_combine(indent, edge_expr, cut=False, atomic=False):
@@ -348,42 +352,52 @@ def source(spec):
     ms_decl_c = ['  __shared__ float4 Ms4[CHUNK][NPP / 4];',
                  '  float (*Ms)[NPP] = reinterpret_cast<float (*)[NPP]>(Ms4);']
     # ------------------------------------------------------------------------------------------- forward
-    def fwd_kernel(cut, rows=False, groups=1):
+    def fwd_kernel(cut, rows=False):
         """``cut`` (kernel ``conv_fwdc``): the weights are W0·c with a per-edge scalar c, read as W0 and scaled in
         registers (the product is never formed in memory); an edge with c == 0 (padding, or past r_max in a
         neighbour list with a skin) contributes exactly zero, so each chunk of 64 edges is first compacted to its
         edges with c != 0 (ballot, then a per-wave LDS scatter by lane rank) and only those are walked.  Every wave
         of the workgroup builds the same list, so the barriers stay uniform.
 
-        ``groups`` > 1 (kernels ``conv_fwd*p``): that many wave groups per receiver, group i walking the i-th slice of
-        its edges in chunks of GROUP_CHUNK; the chunk count is the longest slice's, so that every wave meets every
-        barrier, and the groups' accumulators are added pairwise in LDS (i + i + half, half = groups / 2, ..., 1)."""
-        G2 = groups > 1
-        base = ("conv_fwdcr" if rows else "conv_fwdc") if cut else "conv_fwd"
-        pf = 1 if G2 else FWD_PREFETCH
-        ms = 'Ms4s[grp]' if G2 else 'Ms4'
+        A workgroup of BLOCK threads walks a receiver's edges itself; one of ``fwd_groups`` x BLOCK threads (with
+        ``fwd_groups_lds`` bytes of dynamic LDS) as that many wave groups, each a slice of them."""
+        groups = fwd_groups(spec)
+        # the two forms' registers together: held to three waves per SIMD (the plain form's own count; 184 VGPRs and
+        # two waves for the 2176-weight layer otherwise) where the accumulators and prefetches leave room for it
+        occ = '__attribute__((amdgpu_waves_per_eu(3))) ' if groups and no + 2 * (nx + nk) <= 130 else ''
         F = [
-            f'extern "C" __global__ __launch_bounds__({f"{groups} * BLOCK" if G2 else "BLOCK"}) void '
-            f'{spec.kname(base + ("p" if G2 else ""))}(',
+            f'extern "C" __global__ __launch_bounds__({max(1, groups)} * BLOCK) {occ}void '
+            f'{spec.kname(("conv_fwdcr" if rows else "conv_fwdc") if cut else "conv_fwd")}(',
             '    const float* __restrict__ x, const float* __restrict__ Y, const float* __restrict__ W,',
             '    const int* __restrict__ rowptr, const int* __restrict__ eids, const int* __restrict__ senders,',
             '    float* __restrict__ out, int N' + (', const float* __restrict__ cutv, const int* __restrict__ wrow) {'
                                                    if cut else ') {'),
-        ]
-        if G2:
-            F += [f'  __shared__ float4 Ms4s[{groups}][{GROUP_CHUNK}][NPP / 4];',
-                  f'  __shared__ float red[{groups // 2}][{no}][BLOCK];']
-            F += [f'  __shared__ int sidxs[{groups}][NCB][{GROUP_CHUNK}];'] if cut else []
-        else:
-            F += ms_decl_c + (['  __shared__ int sidx[NCB][CHUNK];'] if cut else [])
-        F += [
+        ] + ['  __shared__ float4 Ms4s[CHUNK][NPP / 4];'] + (['  __shared__ int sidxs[NCB][CHUNK];'] if cut else []) + [
             '  const int n = mh_xcd_block(blockIdx.x, gridDim.x);',
             '  if (n >= N) return;',
-        ] + G.prelude(groups)
+        ]
+        if groups:
+            F += ['  if (blockDim.x == BLOCK) {'] + ['  ' + t for t in fwd_walk(cut, rows, 1)] + ['  } else {']
+            F += ['  ' + t for t in fwd_walk(cut, rows, groups)] + ['  }']
+        else:
+            F += fwd_walk(cut, rows, 1)
+        return F + ['}', '']
+
+    def fwd_walk(cut, rows, groups):
+        """The body of a forward kernel for ``groups`` wave groups per receiver: group i walks the i-th slice of the
+        edges; the chunk count is the longest slice's, so that every wave meets every barrier, and the groups'
+        accumulators are added pairwise in LDS (i + i + half, half = groups / 2, ..., 1)."""
+        G2 = groups > 1
+        pf = 1 if G2 else FWD_PREFETCH
+        ch = chunk_edges(G.npp) // groups
+        F = G.prelude(groups)
+        F += [f'  float4 (*Ms4)[NPP / 4] = Ms4s{f" + grp * {ch}" if G2 else ""};',
+              '  float (*Ms)[NPP] = reinterpret_cast<float (*)[NPP]>(Ms4);']
+        if cut:
+            F += [f'  int (*sidx)[{ch}] = reinterpret_cast<int (*)[{ch}]>(&sidxs[0][0]){" + grp * NCB" if G2 else ""};']
         if G2:
-            F += [f'  float4 (*Ms4)[NPP / 4] = {ms};',
-                  '  float (*Ms)[NPP] = reinterpret_cast<float (*)[NPP]>(Ms4);']
-            F += [f'  int (*sidx)[{GROUP_CHUNK}] = sidxs[grp];'] if cut else []
+            F += ['  extern __shared__ float red_[];            // the upper half\'s accumulators',
+                  f'  float (*red)[{no}][BLOCK] = reinterpret_cast<float (*)[{no}][BLOCK]>(red_);']
         F += [
             '  ' + decl('acc', no, '0.0f'),
             '  ' + decl('xn', nx), '  ' + decl('wn', nk),
@@ -392,9 +406,9 @@ def source(spec):
             F += ['  const int q0 = rowptr[n], q1 = rowptr[n + 1];',
                   f'  const int per = (q1 - q0 + {groups - 1}) / {groups};      // edges of a slice (the last may be shorter)',
                   '  const int p0 = min(q0 + grp * per, q1), p1 = min(p0 + per, q1);',
-                  f'  for (int c0 = 0; c0 < per; c0 += {GROUP_CHUNK}) {{',
+                  f'  for (int c0 = 0; c0 < per; c0 += {ch}) {{',
                   '    const int pb = p0 + c0;',
-                  f'    const int cnt0 = max(0, min({GROUP_CHUNK}, p1 - pb));']
+                  f'    const int cnt0 = max(0, min({ch}, p1 - pb));']
         else:
             F += ['  const int p0 = rowptr[n], p1 = rowptr[n + 1];',
                   '  for (int pb = p0; pb < p1; pb += CHUNK) {',
@@ -458,12 +472,9 @@ def source(spec):
               '    float* __restrict__ o = out + (size_t)n * OUT_DIM;']
         for co in spec.coef:
             F += [f'    mh_st(o + {co["o3"] + c}, ol{co["d3"]}, acc{G.oi[co["k"]] + c});' for c in range(co['d3'])]
-        return F + ['  }', '}', '']
+        return F + ['  }']
 
     L += fwd_kernel(False) + fwd_kernel(True) + fwd_kernel(True, rows=True)
-    if fwd_groups(spec):
-        for kw in (dict(cut=False), dict(cut=True), dict(cut=True, rows=True)):
-            L += fwd_kernel(**kw, groups=FWD_GROUPS)
     # ----------------------------------------------------------------------------------- fused backward
     L += [
         f'extern "C" __global__ __launch_bounds__(BLOCK) void {spec.kname("conv_bwd")}(',
