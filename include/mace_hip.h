@@ -115,7 +115,9 @@ enum mh_kernel_kind {
     MH_EDGE_BWD = 76,    /* the harmonics' and the embedding's backward in one pass                      */
     MH_MLP_BWD_P = 77,   /* radial MLP backward over shared rows, an edge's and its partner's gW0 summed   */
     MH_LIN_BWD_SUM = 78, /* node linear backward over the sum of three gradients of its output               */
-    MH_NUM_KINDS = 79
+    MH_MLP_H3T = 79,     /* radial MLP: derivative of the last hidden activations in the edge length           */
+    MH_CONV_BWD_T = 80,  /* convolution backward to the lengths: gY, dL/dlength, dX messages, no dL/dW         */
+    MH_NUM_KINDS = 81
 };
 
 /* flags of mh_conv_bwd */
@@ -601,6 +603,33 @@ int mh_edge_fwd(mh_module* m, const float* pos, const int32_t* send, const int32
                 float* vec, float* len, float* Y, float* feats, float* cutoff, int64_t E, void* stream);
 int mh_edge_bwd(mh_module* m, const float* vec, const float* len, const float* gY, const float* gfeats,
                 const float* gcutoff, float* gvec, float* glen, int64_t E, void* stream);
+/* mh_edge_fwd that also writes the embedding's derivatives in the length: dfeats [E, n] and dcutoff [E] (both NULL:
+ * mh_edge_fwd). */
+int mh_edge_fwd_tan(mh_module* m, const float* pos, const int32_t* send, const int32_t* recv, const float* shifts,
+                    float* vec, float* len, float* Y, float* feats, float* cutoff, float* dfeats, float* dcutoff,
+                    int64_t E, void* stream);
+/* mh_edge_bwd2 with up to two gradients of the lengths themselves (glen1, glen2 [E], each may be NULL; glen2 needs
+ * glen1), added to what gfeats and gcutoff bring; here gfeats may be NULL too (with gfeats2). */
+int mh_edge_bwd_len(mh_module* m, const float* vec, const float* len, const float* gY, const float* gfeats,
+                    const float* gcutoff, const float* gY2, const float* gfeats2, const float* gcutoff2,
+                    const float* glen1, const float* glen2, float* gvec, float* glen, int64_t E, void* stream);
+/* The radial MLP's derivative in the edge length r, for features that are a function of r alone (dfeats [E, n]: their
+ * derivatives): slot i < count[0] (edge rows[i]; both NULL: every edge) writes d(last hidden activations)/dr to t3
+ * [E, 64] at row i (byrow: at row rows[i]).  mh_mlp_out runs the output layer over such rows in slot order (MH_MLP_OUT, as
+ * mh_mlp_fwd_ws does over its h3): rows of dW0/dr.  The gradient of an edge's length is then the dot product of its
+ * dL/d(W0 c) row with c dW0/dr + c' W0, and that row is never stored (mh_conv_bwd_len).  No reference counterpart. */
+int mh_mlp_tangents(mh_module* m, const float* ef, const float* dfeats, const float* WhT, float* t3, int64_t E,
+                    const int32_t* rows, const int32_t* count, int32_t byrow, void* stream);
+int mh_mlp_out(mh_module* m, const float* h, const uint16_t* Wo, float* W, int64_t E, const int32_t* rows,
+               const int32_t* count, int32_t ncb, void* stream);
+/* The receiver-ordered backward with masked edges (mh_conv_bwd_recv_rows, MH_CUT_MASKED) taken to the edge lengths: W and
+ * T hold the rows of W0 and dW0/dr that edge e reads at wrow[e] (NULL: row e), cutoff and dcutoff [E] are c(r) and c'(r).
+ * Writes gY [E, Y_DIM] and glen[e] = sum_k,u dL/d(W0 c)[e, k, u] (c T + c' W) and, with flags MH_WANT_GX, gx through the
+ * messages `work`.  dL/dW0 is not formed.  No reference counterpart. */
+int mh_conv_bwd_len(mh_module* m, const float* x, const float* g, const float* Y, const float* W, const float* T,
+                    const int32_t* rowptr_r, const int32_t* eids_r, const int32_t* senders, const int32_t* rowptr_s,
+                    const int32_t* eids_s, float* work, float* gx, float* gY, float* glen, const float* cutoff,
+                    const float* dcutoff, const int32_t* wrow, int32_t N, int32_t flags, void* stream);
 /* mh_edge_bwd for outputs that two consumers read: gY2 [E, DIM], gfeats2 [E, n] and gcutoff2 [E] (each may be NULL)
  * are a second consumer's gradients of the same outputs, added to the first's per element (gY + gY2, ...) before
  * use, so that no separate sum of the two runs (the results are those of mh_edge_bwd on the sums).  No reference

@@ -290,6 +290,20 @@ int mh_module_bind(mh_module* m, int kind, const char* name, int block_threads, 
 
 namespace {
 
+// The weight-stationary output layer on a persistent grid: 8 equal per-XCD shares of workgroups (blocks go round-robin
+// over the XCDs), each share a multiple of the ncg = ceil(ncb / 4) column groups, about as many as are resident at once.
+int mlp_out_launch(mh_module* m, const float* h, const uint16_t* Wo, float* W, int64_t E, const int32_t* rows,
+                   const int32_t* count, int32_t ncb, void* stream, const char* what) {
+    const int kind = MH_MLP_OUT;
+    if (!m->k[kind].fn) return fail(-1, std::string(what) + ": kernel slot not bound in this module");
+    int res = 0;
+    if (int rc = resident_blocks(m, kind, &res)) return rc;
+    const int ncg = (ncb + 3) / 4;
+    const int per_xcd = std::max(ncg, (res / 8) / ncg * ncg);
+    void* args[] = {&h, &Wo, &W, &E, &rows, &count};
+    return launch_blocks(m, kind, 8LL * per_xcd, args, stream, what);
+}
+
 // Whether the convolution forward over N receivers runs in its grouped form (four wave groups per receiver, each a
 // quarter of its edges): where that is bound and its workgroups do not fill the device more than 1.6 times over.  A
 // receiver's edges are one serial chain in the plain form, so few receivers leave the chip idle; many receivers fill
@@ -338,6 +352,25 @@ int mh_conv_fwd_cut(mh_module* m, const float* x, const float* Y, const float* W
                     const int32_t* eids, const int32_t* senders, const float* cutoff, float* out, int32_t N,
                     void* stream) {
     return mh_conv_fwd_cut_rows(m, x, Y, W, rowptr, eids, senders, cutoff, nullptr, out, N, stream);
+}
+
+int mh_conv_bwd_len(mh_module* m, const float* x, const float* g, const float* Y, const float* W, const float* T,
+                    const int32_t* rowptr_r, const int32_t* eids_r, const int32_t* senders, const int32_t* rowptr_s,
+                    const int32_t* eids_s, float* work, float* gx, float* gY, float* glen, const float* cutoff,
+                    const float* dcutoff, const int32_t* wrow, int32_t N, int32_t flags, void* stream) {
+    if (!x || !g || !Y || !W || !T || !gY || !glen || !cutoff || !dcutoff)
+        return fail(-1, "mh_conv_bwd_len: NULL operand");
+    const bool want_gx = (flags & MH_WANT_GX) != 0;
+    if (want_gx && (!gx || !work || !rowptr_s || !eids_s))
+        return fail(-1, "mh_conv_bwd_len: gx requested but gx, work or the sender CSR is NULL");
+    int32_t kflags = (want_gx ? 1 : 0) | 2;
+    void* args[] = {&x, &g, &Y, &W, &rowptr_r, &eids_r, &senders, &T, &gY, &work, &N, &kflags, &cutoff, &glen, &wrow,
+                    &dcutoff};
+    int rc = launch(m, MH_CONV_BWD_T, N, args, stream, "mh_conv_bwd_len", bwd_parts(m, MH_CONV_BWD_T, N));
+    if (rc || !want_gx) return rc;
+    const float* msg = work;
+    void* args2[] = {&msg, &rowptr_s, &eids_s, &gx, &N, &cutoff};
+    return launch(m, MH_CONV_GXSUM, N, args2, stream, "mh_conv_bwd_len (dX sum)");
 }
 
 int mh_conv_bwd(mh_module* m, const float* x, const float* g, const float* Y, const float* W,
@@ -834,15 +867,26 @@ int mh_mlp_fwd_ws(mh_module* m, const float* ef, const float* WhT, const uint16_
     if (!m) return fail(-1, "mh_mlp_fwd_ws: null module");
     void* a1[] = {&ef, &WhT, &h3, &E, &rows, &count};
     if (int rc = launch(m, MH_MLP_H3, E, a1, stream, "mh_mlp_fwd_ws (hidden layers)")) return rc;
-    // persistent grid: 8 equal per-XCD shares of workgroups (blocks go round-robin over the XCDs), each share a
-    // multiple of the ncg = ceil(ncb / 4) column groups, about as many as are resident at once
-    if (!m->k[MH_MLP_OUT].fn) return fail(-1, "mh_mlp_fwd_ws: kernel slot MH_MLP_OUT not bound in this module");
-    int res = 0;
-    if (int rc = resident_blocks(m, MH_MLP_OUT, &res)) return rc;
-    const int ncg = (ncb + 3) / 4;
-    const int per_xcd = std::max(ncg, (res / 8) / ncg * ncg);
-    void* a2[] = {&h3, &Wo, &W0, &E, &rows, &count};
-    return launch_blocks(m, MH_MLP_OUT, 8LL * per_xcd, a2, stream, "mh_mlp_fwd_ws (output layer)");
+    return mlp_out_launch(m, h3, Wo, W0, E, rows, count, ncb, stream, "mh_mlp_fwd_ws (output layer)");
+}
+
+int mh_mlp_tangents(mh_module* m, const float* ef, const float* dfeats, const float* WhT, float* t3, int64_t E,
+                    const int32_t* rows, const int32_t* count, int32_t byrow, void* stream) {
+    if (E > 0 && (!ef || !dfeats || !WhT || !t3)) return fail(-1, "mh_mlp_tangents: NULL operand");
+    if ((rows == nullptr) != (count == nullptr)) return fail(-1, "mh_mlp_tangents: rows and count go together");
+    if (E <= 0) return 0;
+    void* args[] = {&ef, &dfeats, &WhT, &t3, &E, &rows, &count, &byrow};
+    return launch(m, MH_MLP_H3T, E, args, stream, "mh_mlp_tangents");
+}
+
+int mh_mlp_out(mh_module* m, const float* h, const uint16_t* Wo, float* W, int64_t E, const int32_t* rows,
+               const int32_t* count, int32_t ncb, void* stream) {
+    if (E > 0 && (!h || !Wo || !W)) return fail(-1, "mh_mlp_out: NULL operand");
+    if ((rows == nullptr) != (count == nullptr)) return fail(-1, "mh_mlp_out: rows and count go together");
+    if (ncb < 1) return fail(-1, "mh_mlp_out: ncb must be positive");
+    if (E <= 0) return 0;
+    if (!m) return fail(-1, "mh_mlp_out: null module");
+    return mlp_out_launch(m, h, Wo, W, E, rows, count, ncb, stream, "mh_mlp_out");
 }
 
 int mh_mlp_fwd(mh_module* m, const float* ef, const float* Wh, const uint16_t* Wl, float* W0, int64_t E, void* stream) {
@@ -1020,20 +1064,36 @@ int mh_emb_bwd(mh_module* m, const float* len, const float* gfeats, const float*
     return launch(m, MH_EMB_BWD, E, args, stream, "mh_emb_bwd");
 }
 
-int mh_edge_fwd(mh_module* m, const float* pos, const int32_t* send, const int32_t* recv, const float* shifts,
-                float* vec, float* len, float* Y, float* feats, float* cutoff, int64_t E, void* stream) {
+int mh_edge_fwd_tan(mh_module* m, const float* pos, const int32_t* send, const int32_t* recv, const float* shifts,
+                    float* vec, float* len, float* Y, float* feats, float* cutoff, float* dfeats, float* dcutoff,
+                    int64_t E, void* stream) {
     if (E > 0 && (!pos || !send || !recv || !shifts || !vec || !len || !Y || !feats || !cutoff))
         return fail(-1, "mh_edge_fwd: NULL operand");
-    void* args[] = {&pos, &send, &recv, &shifts, &vec, &len, &Y, &feats, &cutoff, &E};
+    if ((dfeats == nullptr) != (dcutoff == nullptr)) return fail(-1, "mh_edge_fwd: dfeats and dcutoff go together");
+    void* args[] = {&pos, &send, &recv, &shifts, &vec, &len, &Y, &feats, &cutoff, &E, &dfeats, &dcutoff};
     return launch(m, MH_EDGE_FWD, E, args, stream, "mh_edge_fwd");
+}
+
+int mh_edge_fwd(mh_module* m, const float* pos, const int32_t* send, const int32_t* recv, const float* shifts,
+                float* vec, float* len, float* Y, float* feats, float* cutoff, int64_t E, void* stream) {
+    return mh_edge_fwd_tan(m, pos, send, recv, shifts, vec, len, Y, feats, cutoff, nullptr, nullptr, E, stream);
+}
+
+int mh_edge_bwd_len(mh_module* m, const float* vec, const float* len, const float* gY, const float* gfeats,
+                    const float* gcutoff, const float* gY2, const float* gfeats2, const float* gcutoff2,
+                    const float* glen1, const float* glen2, float* gvec, float* glen, int64_t E, void* stream) {
+    if (E > 0 && (!vec || !len || !gY || !gvec || !glen)) return fail(-1, "mh_edge_bwd: NULL operand");
+    if ((glen2 && !glen1) || (gfeats2 && !gfeats)) return fail(-1, "mh_edge_bwd: a second gradient without a first");
+    void* args[] = {&vec, &len, &gY, &gfeats, &gcutoff, &gvec, &glen, &E, &gY2, &gfeats2, &gcutoff2, &glen1, &glen2};
+    return launch(m, MH_EDGE_BWD, E, args, stream, "mh_edge_bwd");
 }
 
 int mh_edge_bwd2(mh_module* m, const float* vec, const float* len, const float* gY, const float* gfeats,
                  const float* gcutoff, const float* gY2, const float* gfeats2, const float* gcutoff2, float* gvec,
                  float* glen, int64_t E, void* stream) {
-    if (E > 0 && (!vec || !len || !gY || !gfeats || !gvec || !glen)) return fail(-1, "mh_edge_bwd: NULL operand");
-    void* args[] = {&vec, &len, &gY, &gfeats, &gcutoff, &gvec, &glen, &E, &gY2, &gfeats2, &gcutoff2};
-    return launch(m, MH_EDGE_BWD, E, args, stream, "mh_edge_bwd");
+    if (E > 0 && !gfeats) return fail(-1, "mh_edge_bwd: NULL operand");
+    return mh_edge_bwd_len(m, vec, len, gY, gfeats, gcutoff, gY2, gfeats2, gcutoff2, nullptr, nullptr, gvec, glen, E,
+                           stream);
 }
 
 int mh_edge_bwd(mh_module* m, const float* vec, const float* len, const float* gY, const float* gfeats,

@@ -27,7 +27,7 @@ MH_CONV_FWD, MH_CONV_BWD, MH_CONV_BWD_WY, MH_SC_FWD, MH_SC_BWD, MH_CONV_BWD_R, M
     MH_SC_BWD_SI, MH_NL_SETUP, MH_NL_ZERO, MH_NL_BINS, MH_NL_SCAN, MH_NL_PLACE, MH_NL_COUNT, MH_NL_OFFSETS, \
     MH_NL_FILL, MH_SPECIES_ORDER, MH_MLP_JVP, MH_MLP_BWD2, MH_GEOM_SEGSUM, MH_NL_BASES, MH_EDGE_COUNT, \
     MH_EDGE_PLACE, MH_GEOM_SEGSUM1, MH_EDGE_PAIR, MH_CONV_FWD_CR, MH_MLP_H3, MH_MLP_OUT, MH_EDGE_FWD, \
-    MH_EDGE_BWD, MH_MLP_BWD_P, MH_LIN_BWD_SUM = range(79)
+    MH_EDGE_BWD, MH_MLP_BWD_P, MH_LIN_BWD_SUM, MH_MLP_H3T, MH_CONV_BWD_T = range(81)
 MH_WANT_GX, MH_WANT_GWY, MH_CUT_MASKED, MH_CUT_NOZERO = 1, 2, 4, 8
 ABI_VERSION = 43
 
@@ -83,6 +83,11 @@ _SIGS = {
     'mh_edge_fwd': (ctypes.c_int, [_P] * 10 + [ctypes.c_int64, _P]),
     'mh_edge_bwd': (ctypes.c_int, [_P] * 8 + [ctypes.c_int64, _P]),
     'mh_edge_bwd2': (ctypes.c_int, [_P] * 11 + [ctypes.c_int64, _P]),
+    'mh_edge_fwd_tan': (ctypes.c_int, [_P] * 12 + [ctypes.c_int64, _P]),
+    'mh_edge_bwd_len': (ctypes.c_int, [_P] * 13 + [ctypes.c_int64, _P]),
+    'mh_mlp_tangents': (ctypes.c_int, [_P] * 5 + [ctypes.c_int64, _P, _P, _I, _P]),
+    'mh_mlp_out': (ctypes.c_int, [_P] * 4 + [ctypes.c_int64, _P, _P, _I, _P]),
+    'mh_conv_bwd_len': (ctypes.c_int, [_P] * 18 + [_I, _I, _P]),
     'mh_perm_fwd': (ctypes.c_int, [_P] * 3 + [ctypes.c_int, _P]),
     'mh_perm_bwd': (ctypes.c_int, [_P] * 3 + [ctypes.c_int, _P]),
     'mh_geom_fwd': (ctypes.c_int, [_P] * 7 + [ctypes.c_int64, _P]),

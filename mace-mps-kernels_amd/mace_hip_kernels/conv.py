@@ -798,6 +798,10 @@ PAIR_RADIAL = True
 # the patched geometry's lengths, shifts without gradient), the MLP's backward projects each shared row once from the
 # pair's summed dL/dW0 (conv_mlp.ConvRadialFn, mh_mlp_bwd_pairs)
 PAIR_GRADS = True
+# ... and, when the patched edge pass also made the features' derivatives in the length, dL/dW0 is not formed at all:
+# the MLP's backward forms the rows' derivatives in the length, and the convolution's reduces each edge's dL/dlength
+# against them (mh_mlp_tangents, mh_conv_bwd_len)
+LENGTH_GRADS = True
 
 
 def support_pairs(ef, cut, gr, vec=None):
@@ -1027,6 +1031,7 @@ class HipConvTP(torch.nn.Module):
                 _native.MH_CONV_FWD_C: (self.spec.kname('conv_fwdc'), self.spec.block, 1),
                 _native.MH_CONV_FWD_CR: (self.spec.kname('conv_fwdcr'), self.spec.block, 1),
                 _native.MH_CONV_GXSUM: (self.spec.kname('conv_gxsum'), gxsum_block(self.spec), 1),
+                _native.MH_CONV_BWD_T: (self.spec.kname('conv_bwdt'), self.spec.block, 1),
             })
             groups = fwd_groups(self.spec)
             if groups:
@@ -1080,7 +1085,7 @@ class HipConvTP(torch.nn.Module):
         return self._fused_mlp[0] if self._fused_mlp else None
 
     def forward(self, node_feats, edge_attrs, tp_weights, edge_index):
-        from .conv_mlp import ConvMLPFn, ConvRadialFn, FusedWeights
+        from .conv_mlp import ConvMLPFn, ConvRadialFn, FusedWeights, length_tangents
         from .edgefeat import slot
         # the patched edge pass's outputs shared by several convolutions: this one reads aliases with gradient slots
         # of their own where the pass left them (their gradients then need no separate sum)
@@ -1093,7 +1098,7 @@ class HipConvTP(torch.nn.Module):
             if tp_weights.mlp is self.deferred_mlp():
                 # the MLP's kernels and this convolution's in one node: rows outside the cutoff's support skipped
                 return ConvRadialFn.apply(node_feats, edge_attrs, slot(tp_weights.ef), slot(tp_weights.cut),
-                                          edge_index, self)
+                                          edge_index, self, *length_tangents(tp_weights, self.deferred_mlp()))
             tp_weights = tp_weights.value()
         if isinstance(tp_weights, CutoffProduct):
             # the radial MLP's output times the cutoff, never formed: the kernels take the two factors

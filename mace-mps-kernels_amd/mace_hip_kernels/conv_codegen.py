@@ -50,6 +50,10 @@ FENCE_M = True
 W_NT = True
 W_NT_ROWS = False
 W_NT_BWD = True
+# The backward to the lengths (conv_bwdt) reads each shared row of W and of T twice, but further apart than the caches
+# hold: 1280 weights, 39k rows, 232 us with non-temporal loads, 264 cacheable; rows of at most GW_CACHE_NW weights fit
+# the Infinity Cache: 512 weights 75 us cacheable, 80 non-temporal.
+W_NT_TAN = True
 # Store the gW (or ∂/∂W0) rows with the non-temporal policy (written once here; the radial MLP's backward reads
 # them next).  Measured on config 2's captured E+F call: cacheable stores made it 25 us slower.
 GW_NT = True
@@ -130,9 +134,9 @@ class _Gen:
             L += [f'{ind}  {dst}{self.xi[b] + m} = mh_ld(xs + {off + m}, ol{d});' for m in range(d)]
         return L + [f'{ind}}}']
 
-    def ld_w(self, ind, e, dst, nt):
+    def ld_w(self, ind, e, dst, nt, src='W'):
         ld = 'mh_ld_nt' if nt else 'mh_ld'
-        return ([f'{ind}{{ const float* __restrict__ we = W + (size_t)({e}) * NW;'] +
+        return ([f'{ind}{{ const float* __restrict__ we = {src} + (size_t)({e}) * NW;'] +
                 [f'{ind}  {dst}{k} = {ld}(we + {k * self.s.mul}, ol1);' for k in range(self.s.nins)] + [f'{ind}}}'])
 
     def ld_g(self, ind, r, dst):
@@ -228,13 +232,17 @@ class _Gen:
                 L.append(f'{ind}}}')
                 continue
             gw = _sum([f'xv{self.xi[i1] + a} * h{a}' for a in hs])
-            if cut:
+            if cut == 'tan':
+                L += [f'{ind}  const float gwk = {gw};', f'{ind}  Pt = fmaf(gwk, t{k}, Pt);']
+                L.append(f'{ind}  Pc = fmaf(gwk, w0{k}, Pc);' + (' asm volatile("" : "+v"(Pc), "+v"(Pt));' if BWD_PC_FENCE else ''))
+            elif cut:
                 L.append(f'{ind}  const float gwk = {gw};')
                 L.append(f'{ind}  Pc = fmaf(gwk, w0{k}, Pc);' + (' asm volatile("" : "+v"(Pc));' if BWD_PC_FENCE else ''))
                 gw = 'gwk * ce'
             gw_nt = GW_NT and s.nins * s.mul > GW_CACHE_NW
             st = f'{"mh_st_nt" if gw_nt else "mh_st"}(gwe + {k * s.mul}, ol1, {gw});'
-            L.append(f'{ind}  {st}' if self.full else f'{ind}  if (active) {st}')
+            if cut != 'tan':
+                L.append(f'{ind}  {st}' if self.full else f'{ind}  if (active) {st}')
             for b in range(co['d2']):
                 ts = [f'{_lit(v)} * xv{self.xi[i1] + a} * gv{self.oi[k] + c}'
                       for a, bb, c, v in co['terms'] if bb == b]
@@ -558,11 +566,12 @@ def source(spec):
     L += ['}', '']
     L += _bwd_recv(G, gyr, pdecl, decl, copy)
     L += _bwd_recv(G, gyr, pdecl, decl, copy, cut=True)
+    L += _bwd_recv(G, gyr, pdecl, decl, copy, cut=True, tan=True)
     L += _gx_sum(spec)
     return '\n'.join(L)
 
 
-def _bwd_recv(G, gyr, pdecl, decl, copy, cut=False):
+def _bwd_recv(G, gyr, pdecl, decl, copy, cut=False, tan=False):
     """Receiver-ordered backward (rows = receivers, the forward's CSR).  g[r] is loaded once per row and stays in
     registers; each edge gathers only x[s] (X_DIM floats) and its W row, writes its gW row and gY, and, when dX is
     wanted, its dX message gxm[e] = Σ_k W_k·h_k (X_DIM floats), which ``conv_gxsum`` adds up per sender.  Per edge
@@ -580,19 +589,24 @@ def _bwd_recv(G, gyr, pdecl, decl, copy, cut=False):
     gY and ∂/∂c rows for such an edge without reading W0 or x, writes no dX message (``conv_gxsum`` skips the edge
     too), and walks only the other edges of each chunk (compacted by lane rank, as in ``conv_fwdc``).  With flags
     bit 2 as well the zero ∂/∂W0 rows are not written either: for a caller whose only consumer of ∂/∂W0 (the radial
-    MLP's backward) skips the masked rows itself."""
+    MLP's backward) skips the masked rows itself.
+
+    ``tan`` (kernel ``conv_bwdt``): T holds the rows dW0/dr beside W0's (both read through the row map) and dcv the
+    cutoff's derivatives; instead of ∂/∂W0 and ∂/∂c each edge's dL/dr = Σ_{k,u} gW·(c T + c' W0) is reduced like ∂/∂c
+    above.  Nothing as wide as W0 is stored, and the radial MLP has no backward to run over it."""
     spec, nx, nk = G.s, G.nx, G.s.nins
     atomic = GY_LDS_ATOMIC and spec.ncb == 2
     if atomic:
         gyr = gy_reduce('      ', spec.y_dim, spec.y_pad, atomic=True)
     L = [
-        f'extern "C" __global__ __launch_bounds__(BLOCK) void {spec.kname("conv_bwdrc" if cut else "conv_bwdr")}(',
+        f'extern "C" __global__ __launch_bounds__(BLOCK) void {spec.kname("conv_bwdt" if tan else "conv_bwdrc" if cut else "conv_bwdr")}(',
         '    const float* __restrict__ x, const float* __restrict__ g, const float* __restrict__ Y,',
         '    const float* __restrict__ W, const int* __restrict__ rowptr, const int* __restrict__ eids,',
-        '    const int* __restrict__ senders, float* __restrict__ gW, float* __restrict__ gY,',
+        f'    const int* __restrict__ senders, {"const float* __restrict__ T" if tan else "float* __restrict__ gW"}, '
+        'float* __restrict__ gY,',
         '    float* __restrict__ gxm, int N, int flags' +
-        (', const float* __restrict__ cutv, float* __restrict__ gcut, const int* __restrict__ wrow) {'
-         if cut else ') {'),
+        (', const float* __restrict__ cutv, float* __restrict__ gcut, const int* __restrict__ wrow' +
+         (', const float* __restrict__ dcv) {' if tan else ') {') if cut else ') {'),
         '  __shared__ float part[CHUNK][Y_PAD];' if atomic else '  __shared__ float part[NCB][CHUNK][Y_PAD];',
     ] + ((['  __shared__ float partc[CHUNK];'] if atomic else ['  __shared__ float partc[NCB][CHUNK];']) +
          ['  __shared__ int sidx[NCB][CHUNK];'] if cut else []) + [
@@ -611,14 +625,19 @@ def _bwd_recv(G, gyr, pdecl, decl, copy, cut=False):
         '  __syncthreads();',
     ] if atomic else []) + G.prelude() + [
         '  const bool GX = (flags & 1) != 0;',
-    ] + (['  const bool MASKED = (flags & 2) != 0;',
-          '  const bool ZROWS = (flags & 4) == 0;     // write the zero gW rows of masked edges'] if cut else []) + [
+    ] + (['  const bool MASKED = (flags & 2) != 0;'] if cut else []) + ([
+          '  const bool ZROWS = (flags & 4) == 0;     // write the zero gW rows of masked edges'] if cut and not tan else []) + [
         '  ' + decl('gv', G.no),
     ]
     L += G.ld_g('  ', 'r', 'gv')
-    L += ['  ' + decl('xn', nx), '  ' + decl('wn', nk)]
+    L += ['  ' + decl('xn', nx), '  ' + decl('wn', nk)] + (['  ' + decl('tn', nk)] if tan else [])
     if BWD_PREFETCH > 1:
         L += ['  ' + decl('xm', nx), '  ' + decl('wm', nk)]
+    nt = (W_NT_TAN and spec.nins * spec.mul > GW_CACHE_NW) if tan else W_NT_BWD
+
+    def ld_rows(ind, e, dst='w'):
+        """The weight row (and with ``tan`` its tangent) of edge row ``e``."""
+        return G.ld_w(ind, e, dst + 'n', nt) + (G.ld_w(ind, e, 'tn', nt, 'T') if tan else [])
 
     def chunks(msg):
         C = ['  for (int pb = p0; pb < p1; pb += CHUNK) {']
@@ -637,10 +656,11 @@ def _bwd_recv(G, gyr, pdecl, decl, copy, cut=False):
                   '    const int cnt = __popcll(kept);',
                   '    if (keep) sidx[wave][__popcll(kept & ((1ull << lane) - 1ull))] = my_e;',
                   '    for (unsigned long long d = drop; d; d &= d - 1ull) {',
-                  '      const int ez = mh_bcast(my_e, __builtin_ctzll(d));',
-                  '      float* __restrict__ gz = gW + (size_t)ez * NW;']
-            st = [f'mh_st_nt(gz + {k * spec.mul}, ol1, 0.0f);' for k in range(nk)]
-            C += ['      if (ZROWS) {'] + [f'        {t}' if G.full else f'        if (active) {t}' for t in st] + ['      }']
+                  '      const int ez = mh_bcast(my_e, __builtin_ctzll(d));']
+            if not tan:
+                C += ['      float* __restrict__ gz = gW + (size_t)ez * NW;']
+                st = [f'mh_st_nt(gz + {k * spec.mul}, ol1, 0.0f);' for k in range(nk)]
+                C += ['      if (ZROWS) {'] + [f'        {t}' if G.full else f'        if (active) {t}' for t in st] + ['      }']
             C += ['      if (wave == 0) {',
                   '        if (lane < Y_DIM) gY[(size_t)ez * Y_DIM + lane] = 0.0f;',
                   '        if (lane == 0) gcut[ez] = 0.0f;',
@@ -661,7 +681,7 @@ def _bwd_recv(G, gyr, pdecl, decl, copy, cut=False):
                   '    const int my_w = my_e;']
         C += G.m_prologue('    ', 'my_e')
         C += ['    {', '      const int er0 = mh_bcast(my_w, 0), s0 = mh_bcast(my_s, 0);']
-        C += G.ld_x('      ', 's0', 'xn') + G.ld_w('      ', 'er0', 'wn', W_NT_BWD)
+        C += G.ld_x('      ', 's0', 'xn') + ld_rows('      ', 'er0')
         C += ['    }']
         if BWD_PREFETCH > 1:          # edge 1 (or the last edge again) one stage further out
             C += ['    {', '      const int er1 = mh_bcast(my_w, min(1, cnt - 1)), s1 = mh_bcast(my_s, min(1, cnt - 1));']
@@ -669,6 +689,8 @@ def _bwd_recv(G, gyr, pdecl, decl, copy, cut=False):
             C += ['    }']
         C += ['    for (int j = 0; j < cnt; ++j) {', '      const int e = mh_bcast(my_e, j);']
         C += copy('xv', 'xn', nx)
+        if tan:
+            C += copy('t', 'tn', nk) + ['      const float dce = dcv[e];', '      float Pt = 0.0f;']
         if cut:
             C += ['      const float ce = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(my_c), j));'
                   if BWD_CUT_BCAST else '      const float ce = cutv[e];']
@@ -686,12 +708,12 @@ def _bwd_recv(G, gyr, pdecl, decl, copy, cut=False):
         else:
             C += ['      {', '        const int j1 = min(j + 1, cnt - 1);',
                   '        const int er1 = mh_bcast(my_w, j1), s1 = mh_bcast(my_s, j1);']
-            C += G.ld_x('        ', 's1', 'xn') + G.ld_w('        ', 'er1', 'wn', W_NT_BWD)
+            C += G.ld_x('        ', 's1', 'xn') + ld_rows('        ', 'er1')
             C += ['      }']
-        C += [f'      {pdecl}', '      float* __restrict__ gwe = gW + (size_t)e * NW;']
+        C += [f'      {pdecl}'] + ([] if tan else ['      float* __restrict__ gwe = gW + (size_t)e * NW;'])
         if msg:
             C += ['      ' + decl('gxa', nx, '0.0f')]
-        C += G.bwd_body('      ', with_gx=msg, use_m=True, store=True, cut=cut)
+        C += G.bwd_body('      ', with_gx=msg, use_m=True, store=True, cut='tan' if tan else cut)
         if msg:
             C += ['      {', '        float* __restrict__ gme = gxm + (size_t)e * X_DIM;']
             for b, (l, _, off) in enumerate(spec.in1):
@@ -700,6 +722,8 @@ def _bwd_recv(G, gyr, pdecl, decl, copy, cut=False):
                 C += [f'        {t}' if G.full else f'        if (active) {t}' for t in st]
             C += ['      }']
         C += gyr
+        if tan:
+            C += ['      Pc = fmaf(ce, Pt, dce * Pc);             // dL/dr of this edge, this lane\'s share']
         if cut:
             # all-reduce over the wave (every lane ends with the sum), lane 0 keeps the wave's partial
             C += [f'      Pc += {_xchg("Pc", bit)};' for bit in range(5, -1, -1)]

@@ -668,11 +668,19 @@ class ConvRadialFn(torch.autograd.Function):
     positions), the pairs are the exact reverses and the MLP's backward projects each shared row once, from the
     pair's summed dL/dW0 rows (``mh_mlp_bwd_pairs``): half the projections; the pair's summed dL/d(edge features),
     and so the forces, are those of the per-edge backward to fp32 rounding, while the split between the two edges
-    is not kept (the partner's row is zero).  No double backward: the two-kernel modules take that
+    is not kept (the partner's row is zero).
+
+    With a lengths alias ``ln`` and ``tan`` = (dfeats/dr, dcutoff/dr, the lengths' grad_fn) (``length_tangents``) the
+    gradient goes to the lengths instead of to ef and cut: the weights are a function W0(r) c(r) of each edge's length,
+    so dL/dr[e] = sum_k,u dL/d(W0 c)[e, k, u] (c dW0/dr + c' W0), which the convolution's backward reduces in registers
+    (``conv_bwdt``) against rows of dW0/dr, formed from the hidden layers' derivatives in r by the forward's output
+    kernel, one row per edge and its reverse.  dL/dW0 is neither stored nor projected (1280 weights, 78k edges of 39k
+    rows: the projection's 140 us become 27 + 55).  A backward that wants the gradients of ef or cut themselves (the
+    lengths' own producer not run by it) takes the form above.  No double backward: the two-kernel modules take that
     (``patch_model(double_backward=True)``)."""
 
     @staticmethod
-    def forward(ctx, x, Y, ef, cut, edge_index, op):
+    def forward(ctx, x, Y, ef, cut, edge_index, op, ln=None, tan=None):
         from . import conv as C
         from .geometry import lengths_pair_symmetric
         from .radial import mlp_forward
@@ -716,6 +724,8 @@ class ConvRadialFn(torch.autograd.Function):
         ctx.W0, ctx.rows, ctx.count, ctx.masked, ctx.wrow = W0, rows, count, masked, wrow
         ctx.pairs = (frows, fcount, partner) if partner is not None else None
         ctx.op, ctx.gr, ctx.shapes = op, gr, (ef.shape, cut.shape)
+        ctx.tan = tan if partner is not None else None
+        ctx.ln_shape = None if ln is None else ln.shape
         return out
 
     @staticmethod
@@ -727,8 +737,12 @@ class ConvRadialFn(torch.autograd.Function):
         x, Y, ef, cut = ctx.saved_tensors
         op, gr = ctx.op, ctx.gr
         want_x, want_y, want_ef, want_cut = (C._grad_needed(ctx, i) for i in range(4))
+        none = (None,) * 4
         if not (want_x or want_y or want_ef or want_cut):
-            return None, None, None, None, None, None
+            return (None,) * 4 + none
+        if ctx.tan is not None and _executes(ctx.tan[2]):
+            gx, gY, glen = ConvRadialFn._to_lengths(ctx, g.contiguous(), want_x)
+            return gx, gY if want_y else None, None, None, None, None, glen.view(ctx.ln_shape), None
         compact = ctx.rows is not None
         gx, gY, gW0, gcut = C._conv_grads(op, gr, g.contiguous(), x, Y, None, ctx.W0, cut, want_x,
                                           want_y or want_ef or want_cut, masked=ctx.masked, nozero=compact,
@@ -743,4 +757,52 @@ class ConvRadialFn(torch.autograd.Function):
             gef = _mlp_bwd(op.deferred_mlp(), ef, gW0, ctx.rows, ctx.count)
         ef_shape, cut_shape = ctx.shapes
         return (gx, gY if want_y else None, gef.view(ef_shape) if gef is not None else None,
-                gcut.view(cut_shape) if want_cut else None, None, None)
+                gcut.view(cut_shape) if want_cut else None, *none)
+
+    @staticmethod
+    def _to_lengths(ctx, g, want_x):
+        """(gx or None, gY, dL/dlength [E])."""
+        from .radial import mlp_rows, mlp_tangents
+        x, Y, ef, cut = ctx.saved_tensors
+        op, gr, s = ctx.op, ctx.gr, ctx.op.spec
+        mlp = op.deferred_mlp()
+        rows, count, _ = ctx.pairs
+        dfeats, dcut, _ = ctx.tan
+        E, n = Y.shape[0], x.shape[0]
+        T = mlp_rows(mlp, mlp_tangents(mlp, ef, dfeats, rows, count), rows, count)
+        gx = torch.empty_like(x) if want_x else None
+        gY, glen = torch.empty_like(Y), torch.empty_like(cut)
+        work = torch.empty(E, s.x_dim, device=x.device, dtype=torch.float32) if want_x else None
+        rowptr_r, eids_r = gr.by_recv()
+        rowptr_s, eids_s = gr.by_send() if want_x else (None, None)
+        P = _native.ptr
+        _native.launch(f'conv_bwd[{op.tag}]', _native.load().mh_conv_bwd_len, op.module.handle, P(x), P(g), P(Y),
+                       P(ctx.W0), P(T), P(rowptr_r), P(eids_r), P(gr.send), P(rowptr_s), P(eids_s), P(work), P(gx),
+                       P(gY), P(glen), P(cut), P(dcut), P(ctx.wrow), n, _native.MH_WANT_GX if want_x else 0,
+                       _native.stream_of(x))
+        return gx, gY, glen
+
+
+def length_tangents(w, mlp):
+    """(lengths alias, (dfeats, dcutoff, the lengths' grad_fn)) for ``ConvRadialFn`` on the unformed weights ``w`` (a
+    ``FusedWeights`` of ``mlp``), or nothing where its gradient to the lengths does not apply: fewer edges than the row
+    lists pay for, the pairing switched off, gradients off, lengths whose split between an edge and its reverse matters
+    (``geometry.lengths_pair_symmetric``), an MLP the weight-stationary output kernel does not cover, or no derivatives
+    left by the edge pass (``edgefeat.length_slot``)."""
+    from . import conv as C
+    from .edgefeat import length_slot
+    from .geometry import lengths_pair_symmetric
+    if not (C.LENGTH_GRADS and C.PAIR_GRADS and C.PAIR_RADIAL and torch.is_grad_enabled()
+            and w.cut.numel() >= C.EDGE_COMPACT_MIN and mlp.spec.hs[-2] == 64 and C._support_masked(w.cut)
+            and lengths_pair_symmetric(w.ef) is not None):
+        return ()
+    got = length_slot(w.ef, w.cut)
+    return () if got is None else (got[0], got[1:])
+
+
+def _executes(fn):
+    """Whether the running backward pass executes the autograd node ``fn`` (unanswerable: yes)."""
+    try:
+        return bool(torch._C._will_engine_execute_node(fn))
+    except (RuntimeError, AttributeError):
+        return True

@@ -14,12 +14,14 @@ gradient and dL/dlengths from the embedding's, in one pass (the statements of ``
 Outputs left on a tensor are taken only by the module they were made for, only once, and only while the tensor is
 unmodified (same version); any other call computes as before.
 """
+import weakref
+
 import torch
 
 from . import _native
 from . import edge as _edge
 from . import embedding as _emb
-from .pending import set_slots, slot  # noqa: F401  (slot: the joint node's aliases, handed out)
+from .pending import set_slots, slot, stash_owner  # noqa: F401  (slot: the joint node's aliases, handed out)
 
 BLOCK = 256
 FUSE = True            # run the three forwards (and the two backwards) as one pass where a model allows it
@@ -40,7 +42,8 @@ def source(sh_spec, emb_spec):
     L += [f'extern "C" __global__ __launch_bounds__(BLOCK) void {kname(sh_spec, emb_spec, "edge_fwd")}(',
           '    const float* __restrict__ pos, const int* __restrict__ send, const int* __restrict__ recv,',
           '    const float* __restrict__ shifts, float* __restrict__ vec, float* __restrict__ len,',
-          '    float* __restrict__ Y, float* __restrict__ feats, float* __restrict__ cutoff, long long E) {'] + idx
+          '    float* __restrict__ Y, float* __restrict__ feats, float* __restrict__ cutoff, long long E,',
+          '    float* __restrict__ dfeats = nullptr, float* __restrict__ dcutoff = nullptr) {'] + idx
     L += ['  float vx, vy, vz;',
           '  {                                         // the edge vector and its length (geom_fwd)',
           '    const long long s = send[e], r = recv[e];',
@@ -59,14 +62,18 @@ def source(sh_spec, emb_spec):
           '    const float x = le;']
     L += ind(em['head'], 4) + ['    cutoff[e] = cut;'] + ind(em['fwd'], 4)
     L += [f'    feats[e * {n} + {k}] = f{k};' for k in range(n)]
+    L += ['    if (dfeats) {                           // and their derivatives in the length'] + ind(em['tan'], 6)
+    L += ['      dcutoff[e] = dcut;'] + [f'      dfeats[e * {n} + {k}] = df{k};' for k in range(n)] + ['    }']
     L += ['  }', '}', '']
     # gY2 / gfeats2 / gcut2 (each may be NULL): a second consumer's gradients of the same outputs, added to the
-    # first's per element as autograd would (a + b), so that no separate sum runs
+    # first's per element as autograd would (a + b), so that no separate sum runs; gl1 / gl2 (each may be NULL): two
+    # consumers' gradients of the length itself, added to the embedding's (gfeats NULL: none arrives through it)
     L += [f'extern "C" __global__ __launch_bounds__(BLOCK) void {kname(sh_spec, emb_spec, "edge_bwd")}(',
           '    const float* __restrict__ vec, const float* __restrict__ len, const float* __restrict__ gY,',
           '    const float* __restrict__ gfeats, const float* __restrict__ gcut, float* __restrict__ gvec,',
           '    float* __restrict__ glen, long long E, const float* __restrict__ gY2,',
-          '    const float* __restrict__ gfeats2, const float* __restrict__ gcut2) {'] + idx
+          '    const float* __restrict__ gfeats2, const float* __restrict__ gcut2,',
+          '    const float* __restrict__ gl1 = nullptr, const float* __restrict__ gl2 = nullptr) {'] + idx
     L += ['  {                                         // dL/dvec from the harmonics\' gradient (sh_bwd)',
           '    const float vx = vec[3 * e], vy = vec[3 * e + 1], vz = vec[3 * e + 2];']
     L += ind(sh['head'], 4)
@@ -76,11 +83,15 @@ def source(sh_spec, emb_spec):
     L += [f'      g{c} = ge[{c}] + ge2[{c}];' for c in range(dim)]
     L += ['    } else {'] + [f'      g{c} = ge[{c}];' for c in range(dim)] + ['    }']
     L += ind(sh['bwd'], 4) + ['    gvec[3 * e] = ox; gvec[3 * e + 1] = oy; gvec[3 * e + 2] = oz;', '  }']
-    L += ['  {                                         // dL/dlen from the embedding\'s gradients (emb_bwd)',
+    L += ['  float gl = 0.f;',
+          '  if (gl1) gl = gl1[e];',
+          '  if (gl2) gl += gl2[e];',
+          '  if (!gfeats && !gcut && !gcut2) { glen[e] = gl; return; }',
+          '  {                                         // dL/dlen from the embedding\'s gradients (emb_bwd)',
           '    const float x = len[e];']
     L += [f'    float {", ".join(f"gf{k}" for k in range(n))};', '    if (gfeats2) {']
     L += [f'      gf{k} = gfeats[e * {n} + {k}] + gfeats2[e * {n} + {k}];' for k in range(n)]
-    L += ['    } else {'] + [f'      gf{k} = gfeats[e * {n} + {k}];' for k in range(n)] + ['    }']
+    L += ['    } else {'] + [f'      gf{k} = gfeats ? gfeats[e * {n} + {k}] : 0.f;' for k in range(n)] + ['    }']
     L += ['    const bool hc = gcut || gcut2;',
           '    float gc = 0.f;',
           '    if (gcut && gcut2) gc = gcut[e] + gcut2[e];',
@@ -96,7 +107,7 @@ def source(sh_spec, emb_spec):
         bwd.append(new_)
     if hits != n + 1 or any('gfeats' in b or 'gcut' in b for b in bwd):
         raise RuntimeError('edgefeat: the embedding\'s backward statements changed form')
-    L += ind(em['head'] + bwd, 4) + ['    glen[e] = acc;', '  }', '}', '']
+    L += ind(em['head'] + bwd, 4) + ['    glen[e] = gl1 ? acc + gl : acc;', '  }', '}', '']
     return '\n'.join(L)
 
 
@@ -117,9 +128,10 @@ def module(sh_op, emb_op, device):
     return m
 
 
-def forward_all(pos, gr, shifts, vec, ln, ops):
+def forward_all(pos, gr, shifts, vec, ln, ops, tangents=False):
     """Fill vec [E, 3] and ln [E, 1] as ``geom_fwd`` does and leave the harmonics and the embedding of the same edges
-    on ``vec`` for the modules of ``ops`` = (harmonics, embedding)."""
+    on ``vec`` for the modules of ``ops`` = (harmonics, embedding), with the embedding's derivatives in the length
+    (``tangents``) for the convolutions that take the length's gradient themselves (``length_slot``)."""
     sh_op, emb_op = ops
     E = vec.shape[0]
     dev = vec.device
@@ -127,10 +139,12 @@ def forward_all(pos, gr, shifts, vec, ln, ops):
     feats = torch.empty(E, emb_op.spec.n, device=dev, dtype=torch.float32)
     cut = torch.empty(E, 1, device=dev, dtype=torch.float32)
     P = _native.ptr
-    _native.launch(f'edge_fwd[{sh_op.tag}+{emb_op.tag}]', _native.load().mh_edge_fwd,
+    dfeats = torch.empty_like(feats) if tangents else None
+    dcut = torch.empty_like(cut) if tangents else None
+    _native.launch(f'edge_fwd[{sh_op.tag}+{emb_op.tag}]', _native.load().mh_edge_fwd_tan,
                    module(sh_op, emb_op, dev).handle, P(pos), P(gr.send), P(gr.recv), P(shifts), P(vec), P(ln), P(Y),
-                   P(feats), P(cut), E, _native.stream_of(pos))
-    vec._mh_edge = (sh_op, emb_op, ln, Y, feats, cut, vec._version, ln._version)
+                   P(feats), P(cut), P(dfeats), P(dcut), E, _native.stream_of(pos))
+    vec._mh_edge = (sh_op, emb_op, ln, Y, feats, cut, vec._version, ln._version, dfeats, dcut)
 
 
 def _two(gs, shape):
@@ -142,22 +156,23 @@ def _two(gs, shape):
     return gs + [None] * (2 - len(gs))
 
 
-def _edge_bwd(sh_op, emb_op, vec, ln, gYs, gfs, gcs):
-    """(gvec, glen) of the joint node from the gradients its consumers gave each output (lists; None: none)."""
+def _edge_bwd(sh_op, emb_op, vec, ln, gYs, gfs, gcs, gls=()):
+    """(gvec, glen) of the joint node from the gradients its consumers gave each output and the lengths' aliases
+    (lists; None: none)."""
     E = vec.shape[0]
     dev = vec.device
     gY, gY2 = _two(gYs, (E, sh_op.spec.dim))
     gf, gf2 = _two(gfs, (E, emb_op.spec.n))
     gc, gc2 = _two(gcs, (E,))
+    gl1, gl2 = _two(gls, (E,))
     gY = torch.zeros(E, sh_op.spec.dim, device=dev) if gY is None else gY
-    gf = torch.zeros(E, emb_op.spec.n, device=dev) if gf is None else gf
     gv = torch.empty(E, 3, device=dev, dtype=torch.float32)
     gl = torch.empty(E, 1, device=dev, dtype=torch.float32)
     P = _native.ptr
     two = gY2 is not None or gf2 is not None or gc2 is not None
-    _native.launch(f'edge_bwd[{sh_op.tag}+{emb_op.tag}{"+slots" if two else ""}]', _native.load().mh_edge_bwd2,
+    _native.launch(f'edge_bwd[{sh_op.tag}+{emb_op.tag}{"+slots" if two else ""}]', _native.load().mh_edge_bwd_len,
                    module(sh_op, emb_op, dev).handle, P(vec), P(ln), P(gY), P(gf), P(gc), P(gY2), P(gf2), P(gc2),
-                   P(gv), P(gl), E, _native.stream_of(vec))
+                   P(gl1), P(gl2), P(gv), P(gl), E, _native.stream_of(vec))
     return gv, gl
 
 
@@ -166,23 +181,26 @@ class _EdgeFeatFn(torch.autograd.Function):
     that their gradients arrive together and one ``edge_bwd`` serves both.  With ``nslot`` > 0 the node also returns
     ``nslot`` aliases of the three (the same storage, outputs of their own) for the other patched consumers
     (``slot``): each consumer's gradients then reach the node separately, and ``edge_bwd`` adds them as it loads them
-    instead of autograd summing each output's gradients in kernels of their own.  Under create_graph the gradient is
-    the two modules' own differentiable functions (``_SHAdjFn``, ``_EmbAdjFn``) of the summed gradients."""
+    instead of autograd summing each output's gradients in kernels of their own.  After them come ``nlen`` aliases of
+    the lengths, for the consumers that form dL/dlength themselves (``length_slot``): ``edge_bwd`` adds theirs to what
+    the embedding's outputs bring.  Under create_graph the gradient is the two modules' own differentiable functions
+    (``_SHAdjFn``, ``_EmbAdjFn``) of the summed gradients."""
 
     @staticmethod
-    def forward(ctx, vec, ln, made, nslot):
+    def forward(ctx, vec, ln, made, nslot, nlen=0):
         sh_op, emb_op, _, Y, feats, cut = made[:6]
         ctx.save_for_backward(vec, ln)
-        ctx.sh_op, ctx.emb_op = sh_op, emb_op
+        ctx.sh_op, ctx.emb_op, ctx.nslot = sh_op, emb_op, nslot
         extra = []
         for _ in range(nslot):
             extra += [Y.detach(), feats.detach(), cut.detach()]
-        return (Y, feats, cut, *extra)
+        return (Y, feats, cut, *extra, *[ln.detach() for _ in range(nlen)])
 
     @staticmethod
     def backward(ctx, gY, gf, gc, *extra):
         vec, ln = ctx.saved_tensors
         sh_op, emb_op = ctx.sh_op, ctx.emb_op
+        extra, gls = extra[:3 * ctx.nslot], extra[3 * ctx.nslot:]
         gYs, gfs, gcs = [gY, *extra[0::3]], [gf, *extra[1::3]], [gc, *extra[2::3]]
         if torch.is_grad_enabled():          # only true under create_graph=True
             if not sh_op.double_backward:
@@ -193,9 +211,10 @@ class _EdgeFeatFn(torch.autograd.Function):
             gY, gf, gc = total(gYs), total(gfs), total(gcs)
             gv = None if gY is None else _edge._SHAdjFn.apply(gY, vec, sh_op)
             gl = None if gf is None and gc is None else _emb._EmbAdjFn.apply(gf, gc, ln, emb_op)
-            return gv, gl, None, None
-        gv, gl = _edge_bwd(sh_op, emb_op, vec, ln, gYs, gfs, gcs)
-        return gv, gl.reshape(ln.shape), None, None
+            gl = total([gl, *gls])
+            return gv, gl, None, None, None
+        gv, gl = _edge_bwd(sh_op, emb_op, vec, ln, gYs, gfs, gcs, gls)
+        return gv, gl.reshape(ln.shape), None, None, None
 
 
 
@@ -211,13 +230,32 @@ def take_harmonics(sh_op, vec):
     if ln._version != made[7]:
         return None
     nslot = max(0, int(getattr(sh_op, 'slots', 0)))
-    outs = _EdgeFeatFn.apply(vec, ln, made, nslot)
+    nlen = nslot + 1 if made[8] is not None and not sh_op.double_backward else 0
+    outs = _EdgeFeatFn.apply(vec, ln, made, nslot, nlen)
     Y, feats, cut = outs[:3]
     if nslot:
         for k, t in enumerate((Y, feats, cut)):
-            set_slots(t, outs[3 + k::3])
+            set_slots(t, outs[3 + k:3 + 3 * nslot:3])
+    if nlen:
+        # (the lengths' own producer tells a backward whether dL/dlength is wanted at all)
+        feats._mh_len = (feats._version, weakref.ref(cut), cut._version, made[8], made[9], list(outs[-nlen:]), ln.grad_fn)
     ln._mh_emb = (made[1], feats, cut, ln._version)
     return Y
+
+
+def length_slot(feats, cut):
+    """(lengths alias, dfeats/dlength, dcutoff/dlength, the lengths' grad_fn) for a consumer of the joint node's features
+    and cutoff that forms dL/dlength itself (its gradient goes to the alias, none to the features and the cutoff): where
+    the node left one, both tensors are unmodified, and nothing watches their own gradients (a hook, retain_grad);
+    else None."""
+    feats, cut = stash_owner(feats), stash_owner(cut)
+    m = getattr(feats, '_mh_len', None)
+    if (m is None or m[0] != feats._version or m[1]() is not cut or m[2] != cut._version or not m[5]
+            or not m[5][0].requires_grad or m[6] is None):
+        return None
+    if any(t._backward_hooks or t.retains_grad for t in (feats, cut)):
+        return None
+    return m[5].pop(0), m[3], m[4], m[6]
 
 
 def take_embedding(emb_op, ln):

@@ -80,7 +80,8 @@ class EmbSpec:
 
 def math_lines(spec):
     """The per-edge arithmetic as plain C statements of the length ``x``: ``head`` defines the envelope ``cut``,
-    ``fwd`` the features ``f0..f{n-1}``, ``bwd`` (reading ``gfeats`` and ``gcut`` at edge ``e``) ``acc`` = dL/dx."""
+    ``fwd`` the features ``f0..f{n-1}``, ``bwd`` (reading ``gfeats`` and ``gcut`` at edge ``e``) ``acc`` = dL/dx, ``tan``
+    the derivatives ``df0..df{n-1}`` and ``dcut`` of the features and the envelope in x."""
     p, n = spec.p, spec.n
     c1, c2, c3 = (p + 1.0) * (p + 2.0) / 2.0, p * (p + 2.0), p * (p + 1.0) / 2.0
 
@@ -106,7 +107,11 @@ def math_lines(spec):
                 f'  const float db = {_lit(spec.pref)} * ({_lit(w)} * c - s * ix) * ix;',
                 f'  acc += gfeats[e * {n} + {k}] * (db * cut + b * dcut);',
                 '}']
-    return dict(head=head, fwd=fwd, bwd=bwd)
+    tan = bwd[:3] + [f'float {", ".join(f"df{k}" for k in range(n))};']
+    for k, w in enumerate(spec.w):
+        tan += ['{', '  float s, c;', f'  sincosf({_lit(w)} * x, &s, &c);',
+                f'  df{k} = {_lit(spec.pref)} * ({_lit(w)} * c - s * ix) * ix * cut + {_lit(spec.pref)} * s * ix * dcut;', '}']
+    return dict(head=head, fwd=fwd, bwd=bwd, tan=tan)
 
 
 def source(spec):

@@ -229,7 +229,8 @@ class _GeomFn(torch.autograd.Function):
         if edge_ops is not None:
             # the harmonics and the embedding of the same edges in the same pass, left on vec for those modules
             from . import edgefeat
-            edgefeat.forward_all(p, gr, sh, vec, ln, edge_ops)
+            edgefeat.forward_all(p, gr, sh, vec, ln, edge_ops, tangents=ctx.needs_input_grad[0] and _conv.PAIR_GRADS
+                                 and _conv.LENGTH_GRADS and E >= _conv.EDGE_COMPACT_MIN)
         else:
             mod = _module(p.device)
             _native.launch('geom_fwd', _native.load().mh_geom_fwd, mod.handle, _native.ptr(p), _native.ptr(gr.send),

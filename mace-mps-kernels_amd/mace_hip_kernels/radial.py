@@ -263,11 +263,11 @@ def _source(spec, second):
          '__device__ __forceinline__ float mlp_sig(float z) {',
          '  return __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-1.4426950408889634f * z));',
          '}', '']
+    # h = c z s(z) (s the logistic function): h' = c s (1 + z (1 - s)), h'' = c s (1 - s) (2 + z (1 - 2 s))
+    L += ['__device__ __forceinline__ float mlp_d1(float z) { const float s = mlp_sig(z); '
+          'return s * (1.f + z * (1.f - s)); }', '']
     if second:
-        # h = c z s(z) (s the logistic function): h' = c s (1 + z (1 - s)), h'' = c s (1 - s) (2 + z (1 - 2 s))
-        L += ['__device__ __forceinline__ float mlp_d1(float z) { const float s = mlp_sig(z); '
-              'return s * (1.f + z * (1.f - s)); }',
-              '__device__ __forceinline__ float mlp_d2(float z) { const float s = mlp_sig(z); '
+        L += ['__device__ __forceinline__ float mlp_d2(float z) { const float s = mlp_sig(z); '
               'return s * (1.f - s) * (2.f + z * (1.f - 2.f * s)); }', '']
 
     def head(name, args, lds, nb, waves=BLOCK // 64, indexed=False, wpe=None, extra=''):
@@ -746,6 +746,23 @@ def _source(spec, second):
         H += ['  }', '}', '']
         return H
 
+    def h3t_kernel(name):
+        """mlp_bwdp_h: the derivative of ``mlp_h3``'s result in the edge length (the hidden layers on dual numbers, the
+        features ef carrying their derivatives dfe): slot i < count (edge rows[i]) stores dh/dr to ``t3`` at row i, or
+        with ``byrow`` at row rows[i].  The output layer over it gives the derivatives of the W0 rows."""
+        H = head(name, 'const float* __restrict__ ef, const float* __restrict__ dfe, const float* __restrict__ Wh, '
+                 'float* __restrict__ t3, long long E', Lo['tr_size'], 1, indexed=True, extra=', int byrow')
+        H += skip_block(1, zero_rows=False)
+        H += xin(range(1)) + xin(range(1), 'dfe', 'xv')
+        H += stage('Wh', Lo['tr_size']) + ['  __syncthreads();']
+        H += hidden_fwd(True, False, range(1), dual=True, keep_t=True)
+        H += ['  if (do0) {',
+              f'    const long long at = (byrow ? rowc0 : ej0) * {HL};']
+        H += [f'    *reinterpret_cast<mh_f4*>(t3 + at + {32 * st + 4 * tt} + 8 * q) = ht{nh - 1}_0[{2 * st + tt}];'
+              for st in range(S) for tt in range(2)]
+        H += ['  }', '}', '']
+        return H
+
     def out_kernel(name):
         """mlp_out: the output layer over h3, weight-stationary.  A workgroup is 4 waves on 4 consecutive 64-column
         blocks (a column group of 256 columns); each wave keeps its block of the split output layer in registers for
@@ -909,6 +926,7 @@ def _source(spec, second):
         L += bwd_kernel(spec.kname('mlp_bwdp'), False, paired=True)
         hidden_only()
         L += h3_kernel(spec.kname('mlp_h3')) + out_kernel(spec.kname('mlp_out'))
+        L += h3t_kernel(spec.kname('mlp_bwdp_h'))
     return '\n'.join(L)
 
 
@@ -1001,6 +1019,28 @@ def mlp_forward(op, ef, rows=None, count=None):
     return out
 
 
+def mlp_tangents(op, ef, dfeats, rows, count, byrow=False):
+    """dh/dr [E, 64]: the derivative of the listed rows' last hidden activations in the edge length, from the features
+    and their derivatives in it (``mlp_bwdp_h``); at slot i for edge rows[i], or with ``byrow`` at row rows[i]."""
+    E = ef.shape[0]
+    t3 = torch.empty(E, op.spec.hs[-2], device=ef.device, dtype=torch.float32)
+    P = _native.ptr
+    op.bwd_paired = True
+    _native.launch(f'mlp_bwd[{op.tag}]', _native.load().mh_mlp_tangents, op.module.handle, P(ef), P(dfeats), P(op.WhT),
+                   P(t3), E, P(rows), P(count), int(byrow), _native.stream_of(ef))
+    return t3
+
+
+def mlp_rows(op, h, rows, count):
+    """The output layer over h (slot i: edge rows[i]) into rows [E, n_out] (the listed rows only): over
+    ``mlp_tangents``, the derivatives of the W0 rows in the edge length."""
+    out = torch.empty(h.shape[0], op.spec.hs[-1], device=h.device, dtype=torch.float32)
+    P = _native.ptr
+    _native.launch(f'mlp_out[{op.tag}]', _native.load().mh_mlp_out, op.module.handle, P(h), P(op.Wo), P(out),
+                   h.shape[0], P(rows), P(count), op.ncb, _native.stream_of(h))
+    return out
+
+
 class _MLPFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, ef, op):
@@ -1084,6 +1124,7 @@ class HipRadialMLP(torch.nn.Module):
                 _native.MH_MLP_HIDB: (self.spec.kname('mlp_hidb'), BLOCK, 64 * NB_BWD),
                 _native.MH_MLP_H3: (self.spec.kname('mlp_h3'), BLOCK, 64),
                 _native.MH_MLP_OUT: (self.spec.kname('mlp_out'), BLOCK, 1),
+                _native.MH_MLP_H3T: (self.spec.kname('mlp_bwdp_h'), BLOCK, 64),
             })
         self.ncb = -(-self.spec.hs[-1] // WS_COLS)
         pw = packed_weights(self.spec)
