@@ -328,6 +328,17 @@ int bwd_parts(const mh_module* m, int kind, int64_t N) {
     return waves <= 384 ? 8 : waves <= 3072 ? 4 : waves <= 8192 ? 2 : 1;
 }
 
+// The same for the backward to the lengths, whose rows two receivers share: more slices spread the two readers of a row
+// further apart in time, and with enough receivers to fill the device its caches matter more.  Measured in the model,
+// 1280 weights (us, 1 / 2 / 4 per receiver; slabs of about 160 atoms, and bulk): N = 648 98 / 72 / 74, 1626 169 / 159 / 152,
+// 2600 243 / 271 / 273, 3704 339 / 401 / 438, 5100 448 / 548 / 600; bulk 1372 157 / 158 / 160, 4000 498 / 536 / 580, 6912
+// 845 / 924 / 999 (non-temporal loads of the rows, one per receiver: 2600 242, 3704 370, 6912 951).
+int bwd_len_parts(const mh_module* m, int kind, int64_t N) {
+    if (!m) return 1;
+    const int64_t waves = N * (m->k[kind].block / 64);
+    return waves <= 384 ? 8 : waves <= 4096 ? 4 : 1;
+}
+
 }  // namespace
 
 extern "C" {
@@ -366,7 +377,7 @@ int mh_conv_bwd_len(mh_module* m, const float* x, const float* g, const float* Y
     int32_t kflags = (want_gx ? 1 : 0) | 2;
     void* args[] = {&x, &g, &Y, &W, &rowptr_r, &eids_r, &senders, &T, &gY, &work, &N, &kflags, &cutoff, &glen, &wrow,
                     &dcutoff};
-    int rc = launch(m, MH_CONV_BWD_T, N, args, stream, "mh_conv_bwd_len", bwd_parts(m, MH_CONV_BWD_T, N));
+    int rc = launch(m, MH_CONV_BWD_T, N, args, stream, "mh_conv_bwd_len", bwd_len_parts(m, MH_CONV_BWD_T, N));
     if (rc || !want_gx) return rc;
     const float* msg = work;
     void* args2[] = {&msg, &rowptr_s, &eids_s, &gx, &N, &cutoff};

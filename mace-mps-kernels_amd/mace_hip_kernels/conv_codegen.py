@@ -50,10 +50,6 @@ FENCE_M = True
 W_NT = True
 W_NT_ROWS = False
 W_NT_BWD = True
-# The backward to the lengths (conv_bwdt) reads each shared row of W and of T twice, but further apart than the caches
-# hold: 1280 weights, 39k rows, 232 us with non-temporal loads, 264 cacheable; rows of at most GW_CACHE_NW weights fit
-# the Infinity Cache: 512 weights 75 us cacheable, 80 non-temporal.
-W_NT_TAN = True
 # Store the gW (or ∂/∂W0) rows with the non-temporal policy (written once here; the radial MLP's backward reads
 # them next).  Measured on config 2's captured E+F call: cacheable stores made it 25 us slower.
 GW_NT = True
@@ -633,7 +629,7 @@ def _bwd_recv(G, gyr, pdecl, decl, copy, cut=False, tan=False):
     L += ['  ' + decl('xn', nx), '  ' + decl('wn', nk)] + (['  ' + decl('tn', nk)] if tan else [])
     if BWD_PREFETCH > 1:
         L += ['  ' + decl('xm', nx), '  ' + decl('wm', nk)]
-    nt = (W_NT_TAN and spec.nins * spec.mul > GW_CACHE_NW) if tan else W_NT_BWD
+    nt = W_NT_BWD and not tan            # (tan: each shared row of W0 and of T is read twice)
 
     def ld_rows(ind, e, dst='w'):
         """The weight row (and with ``tan`` its tangent) of edge row ``e``."""
