@@ -280,12 +280,14 @@ def launch(tag, fn, *args):
 
 
 def ptr(t):
-    """Device pointer of a tensor (None → NULL)."""
-    return None if t is None else _P(t.data_ptr())
+    """Device pointer of a tensor (None → NULL), for a C-ABI argument declared as a pointer."""
+    return None if t is None else t.data_ptr()
 
 
 def stream_of(t):
-    return _P(torch.cuda.current_stream(t.device).cuda_stream)
+    """The current stream of a GPU tensor's device.  The raw handle: a torch.cuda.Stream object per launch was 3 us of
+    host time, about 100 us of an eager energy and forces call of 34 launches (1.1 ms of host work in all)."""
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 # ------------------------------------------------------------------------------------------- graph capture
@@ -296,7 +298,7 @@ _capture_holds = []
 
 
 def capturing():
-    return torch.cuda.is_available() and torch.cuda.is_current_stream_capturing()
+    return torch.cuda.is_initialized() and torch._C._cuda_isCurrentStreamCapturing()
 
 
 def hold_for_capture(obj):
