@@ -117,7 +117,9 @@ enum mh_kernel_kind {
     MH_LIN_BWD_SUM = 78, /* node linear backward over the sum of three gradients of its output               */
     MH_MLP_H3T = 79,     /* radial MLP: derivative of the last hidden activations in the edge length           */
     MH_CONV_BWD_T = 80,  /* convolution backward to the lengths: gY, dL/dlength, dX messages, no dL/dW         */
-    MH_NUM_KINDS = 81
+    MH_GEOM_STRAIN = 81, /* stress displacement: strained positions and shifts                                 */
+    MH_GEOM_DET = 82,    /* determinants of 3x3 matrices                                                       */
+    MH_NUM_KINDS = 83
 };
 
 /* flags of mh_conv_bwd */
@@ -402,10 +404,30 @@ int mh_geom_jvp(mh_module* m, const float* vec, const float* len, const float* g
  * perm[seg[b + 1] - 1] (perm [M] int32), or rows seg[b] .. seg[b + 1] - 1 with perm NULL (seg [B + 1] int64, g [M, 9],
  * out [B, 9]).  The backward of MACE's per-structure gathers in get_symmetric_displacement (the symmetric strain by
  * atom, the strained cell by edge: segments from the batch's ptr and the sender CSR).  One workgroup per structure
- * (bind MH_GEOM_SEGSUM with 256 threads and rows_per_block 1); fixed summation order.  No reference counterpart. */
+ * (bind MH_GEOM_SEGSUM with 1024 threads and rows_per_block 1); fixed summation order.  No reference counterpart. */
 int mh_geom_segsum(mh_module* m, const float* g, const int32_t* perm, const int64_t* seg, float* out, int32_t B,
                    void* stream);
-/* The same for one column, out[b] = sum of g[seg[b]] .. g[seg[b + 1] - 1] (g [M], seg [B + 1] int64, out [B]):
+/* MACE's get_symmetric_displacement: with sym = (D + D^T) / 2 of structure b (disp [B, 9]), opos = pos + pos sym of an
+ * atom's structure batch[i] (int64; pos, opos [N, 3]) and osh = unit (cell + cell sym) of its sender's (unit, osh
+ * [E, 3], send [E] int32 in 0 .. N - 1, cell [B, 9]).  Bind MH_GEOM_STRAIN with 256 threads and rows_per_block 256.
+ *
+ * mh_geom_strain_sum is one half of its backward: the sum over the rows of segment b of left[row] x g[row] (3 wide
+ * each, the outer product).  Segment b is rows seg[b] .. seg[b + 1] - 1 (seg [B + 1] int64, bounded by n), or, with
+ * rowptr [n + 1] and perm, perm[rowptr[seg[b]]] .. perm[rowptr[seg[b + 1]] - 1].  out [B slices, 9]: each of the
+ * `slices` workgroups of a segment writes its own row.  For the edges: left = unit, g = dL/dosh, the sender CSR.
+ * For the atoms (left = pos, g = dL/dopos, one slice): cell, parts (the edges' [B nparts, 9]) and disp given, out is
+ * dL/ddisp [B, 9] and gleft [n, 3] dL/dpos.  Uses MH_GEOM_SEGSUM.
+ *
+ * mh_geom_det: out[b] = det of the 3x3 matrix a[b] (a [B, 9]), expanded in float64.  Bind MH_GEOM_DET with 256 threads
+ * and rows_per_block 256.  No reference counterparts. */
+int mh_geom_strain(mh_module* m, const float* pos, const float* unit, const float* cell, const float* disp,
+                   const int64_t* batch, const int32_t* send, float* opos, float* osh, int32_t N, int64_t E, int32_t B,
+                   void* stream);
+int mh_geom_strain_sum(mh_module* m, const float* left, const float* g, const int32_t* perm, const int64_t* seg,
+                       const int32_t* rowptr, int32_t n, float* out, int32_t slices, const float* cell,
+                       const float* parts, int32_t nparts, const float* disp, float* gleft, int32_t B, void* stream);
+int mh_geom_det(mh_module* m, const float* a, float* out, int32_t B, void* stream);
+/* The sum of rows (mh_geom_segsum) for one column, out[b] = sum of g[seg[b]] .. g[seg[b + 1] - 1] (g [M], seg [B + 1] int64, out [B]):
  * MACE's per-structure energy sums (scatter_sum of the node energies by the sorted batch vector), deterministic
  * where an atomic index_add is not.  Bind MH_GEOM_SEGSUM1 with 256 threads and rows_per_block 1.  No reference
  * counterpart. */

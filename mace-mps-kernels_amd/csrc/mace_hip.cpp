@@ -146,7 +146,7 @@ extern "C" {
 
 const char* mh_last_error(void) { return g_err.c_str(); }
 
-int mh_version(void) { return 43; }
+int mh_version(void) { return 44; }
 
 int mh_launch_log(int enable) {
     std::lock_guard<std::mutex> lock(g_log_mu);
@@ -798,8 +798,42 @@ int mh_geom_segsum(mh_module* m, const float* g, const int32_t* perm, const int6
                    void* stream) {
     if (B < 0) return fail(-1, "mh_geom_segsum: negative structure count");
     if (B > 0 && (!g || !seg || !out)) return fail(-1, "mh_geom_segsum: NULL operand");
-    void* args[] = {&g, &perm, &seg, &out, &B};
+    const float* none = nullptr;
+    const int32_t* rowptr = nullptr;
+    float* gleft = nullptr;
+    int32_t n = 0, slices = 1, nparts = 0;
+    void* args[] = {&g, &perm, &seg, &out, &B, &none, &rowptr, &n, &slices, &none, &none, &nparts, &none, &gleft};
     return launch(m, MH_GEOM_SEGSUM, B, args, stream, "mh_geom_segsum");
+}
+
+int mh_geom_strain(mh_module* m, const float* pos, const float* unit, const float* cell, const float* disp,
+                   const int64_t* batch, const int32_t* send, float* opos, float* osh, int32_t N, int64_t E, int32_t B,
+                   void* stream) {
+    if (N < 0 || E < 0 || B < 0) return fail(-1, "mh_geom_strain: negative size");
+    if (N > 0 && (B == 0 || !pos || !cell || !disp || !batch || !opos))
+        return fail(-1, "mh_geom_strain: NULL operand or no structures");
+    if (E > 0 && (N == 0 || !unit || !send || !osh)) return fail(-1, "mh_geom_strain: NULL edge operand or no atoms");
+    void* args[] = {&pos, &unit, &cell, &disp, &batch, &send, &opos, &osh, &N, &E, &B};
+    return launch(m, MH_GEOM_STRAIN, E > N ? E : N, args, stream, "mh_geom_strain");
+}
+
+int mh_geom_strain_sum(mh_module* m, const float* left, const float* g, const int32_t* perm, const int64_t* seg,
+                       const int32_t* rowptr, int32_t n, float* out, int32_t slices, const float* cell,
+                       const float* parts, int32_t nparts, const float* disp, float* gleft, int32_t B, void* stream) {
+    if (B < 0 || n < 0 || slices < 1 || nparts < 0) return fail(-1, "mh_geom_strain_sum: bad size");
+    if (static_cast<int64_t>(B) * slices > 0x7fffffff) return fail(-1, "mh_geom_strain_sum: launch too large");
+    if (!left) return n ? fail(-1, "mh_geom_strain_sum: NULL left") : 0;
+    if (B > 0 && (!g || !seg || !out)) return fail(-1, "mh_geom_strain_sum: NULL operand");
+    if (cell && (slices != 1 || nparts < 1 || !parts)) return fail(-1, "mh_geom_strain_sum: bad epilogue");
+    if (gleft && !disp) return fail(-1, "mh_geom_strain_sum: gleft needs disp");
+    void* args[] = {&g, &perm, &seg, &out, &B, &left, &rowptr, &n, &slices, &cell, &parts, &nparts, &disp, &gleft};
+    return launch(m, MH_GEOM_SEGSUM, static_cast<int64_t>(B) * slices, args, stream, "mh_geom_strain_sum");
+}
+
+int mh_geom_det(mh_module* m, const float* a, float* out, int32_t B, void* stream) {
+    if (B > 0 && (!a || !out)) return fail(-1, "mh_geom_det: NULL operand");
+    void* args[] = {&a, &out, &B};
+    return launch(m, MH_GEOM_DET, B, args, stream, "mh_geom_det");
 }
 
 int mh_geom_segsum1(mh_module* m, const float* g, const int64_t* seg, float* out, int32_t B, void* stream) {

@@ -27,9 +27,10 @@ MH_CONV_FWD, MH_CONV_BWD, MH_CONV_BWD_WY, MH_SC_FWD, MH_SC_BWD, MH_CONV_BWD_R, M
     MH_SC_BWD_SI, MH_NL_SETUP, MH_NL_ZERO, MH_NL_BINS, MH_NL_SCAN, MH_NL_PLACE, MH_NL_COUNT, MH_NL_OFFSETS, \
     MH_NL_FILL, MH_SPECIES_ORDER, MH_MLP_JVP, MH_MLP_BWD2, MH_GEOM_SEGSUM, MH_NL_BASES, MH_EDGE_COUNT, \
     MH_EDGE_PLACE, MH_GEOM_SEGSUM1, MH_EDGE_PAIR, MH_CONV_FWD_CR, MH_MLP_H3, MH_MLP_OUT, MH_EDGE_FWD, \
-    MH_EDGE_BWD, MH_MLP_BWD_P, MH_LIN_BWD_SUM, MH_MLP_H3T, MH_CONV_BWD_T = range(81)
+    MH_EDGE_BWD, MH_MLP_BWD_P, MH_LIN_BWD_SUM, MH_MLP_H3T, MH_CONV_BWD_T, \
+    MH_GEOM_STRAIN, MH_GEOM_DET = range(83)
 MH_WANT_GX, MH_WANT_GWY, MH_CUT_MASKED, MH_CUT_NOZERO = 1, 2, 4, 8
-ABI_VERSION = 43
+ABI_VERSION = 44
 
 # hipcc/hipRTC options for every generated layer: gfx950 code, -O3, and packed-FP32 instructions disabled.
 ARCH = os.environ.get('MACE_HIP_ARCH', 'gfx950')
@@ -119,6 +120,9 @@ _SIGS = {
     'mh_sc_bwd2': (ctypes.c_int, [_P] * 7 + [_I, _I, _P]),
     'mh_sc_bwd': (ctypes.c_int, [_P] * 6 + [_I, _P]),
     'mh_geom_segsum': (ctypes.c_int, [_P] * 5 + [_I, _P]),
+    'mh_geom_strain': (ctypes.c_int, [_P] * 9 + [_I, ctypes.c_int64, _I, _P]),
+    'mh_geom_strain_sum': (ctypes.c_int, [_P] * 6 + [_I, _P, _I, _P, _P, _I, _P, _P, _I, _P]),
+    'mh_geom_det': (ctypes.c_int, [_P] * 3 + [_I, _P]),
     'mh_mlp_jvp': (ctypes.c_int, [_P] * 6 + [ctypes.c_int64, _P]),
     'mh_mlp_bwd2': (ctypes.c_int, [_P] * 7 + [ctypes.c_int64, _P]),
     'mh_species_order': (ctypes.c_int, [_P, _P, _I, _I, _P, _P, _P, _I, _I, _P]),

@@ -12,9 +12,12 @@ the same edge_index: deterministic, no atomics, no sort.
 With stress or virials, MACE first strains each structure (``get_symmetric_displacement``): positions + positions
 @ sym[batch] and shifts = unit_shifts @ cell[batch[sender]].  The backward of those two per-structure gathers is, in
 PyTorch, an index_put with accumulation whose runs of equal indices are summed serially: on one structure every
-atom and edge carries the same index and the two take ~1.9 ms of a 2.6 ms E+F+stress call.  Here the gathers stay
-and their backward is a segmented sum per structure (``geom_segsum``; atoms by the batch's ptr, edges by the sender
-CSR), one workgroup per structure in a fixed order.
+atom and edge carries the same index and the two take ~1.9 ms of a 2.6 ms E+F+stress call.  Here the strain is
+one kernel (``geom_strain``) and its backward two segmented sums per structure (``geom_segsum``; edges by the sender
+CSR, atoms by the batch's ptr) in a fixed order, and the volume that the stress is divided by (``torch.linalg.det``
+in MACE's ``get_outputs``) one more (``geom_det``).  A force or stress loss (patched with ``double_backward=True``)
+keeps the gathers as PyTorch expressions around the segmented sums, which differentiate twice.  One captured E+F+stress
+call of 160 atoms, whose launches cost 2 to 3 us each: 494 us with the expressions and torch.linalg.det, 406 so.
 
 MACE's per-structure energy sums (``scatter_sum`` of the node energies by the batch vector) are an index_add with
 float atomics in PyTorch (~9 us each on config 2's 16 structures, and the summation order varies from run to run);
@@ -38,6 +41,9 @@ from . import _native
 from . import conv as _conv
 
 BLOCK = 256
+SEG_BLOCK = 1024          # threads of a segmented sum of 3x3 rows
+SLICE_ROWS = 8192         # edges of a structure per workgroup of that sum (8 per thread), up to MAX_SLICES workgroups
+MAX_SLICES = 64
 _ACTIVE = contextvars.ContextVar('mace_hip_kernels_geometry', default=False)
 _PTR = contextvars.ContextVar('mace_hip_kernels_geometry_ptr', default=None)   # the batch's ptr during a forward
 _BATCH = contextvars.ContextVar('mace_hip_kernels_geometry_batch', default=None)  # the batch vector, likewise
@@ -46,6 +52,7 @@ _EDGE = contextvars.ContextVar('mace_hip_kernels_geometry_edge', default=None)
 FUNCTION = 'get_edge_vectors_and_lengths'
 DISPLACEMENT = 'get_symmetric_displacement'
 SCATTER = 'scatter_sum'
+OUTPUTS = 'get_outputs'
 
 _SOURCE = r'''
 #define BLOCK 256
@@ -131,31 +138,126 @@ extern "C" __global__ __launch_bounds__(BLOCK) void geom_jvp(const float* __rest
   h[3 * e] = c * (dx - ux * ud); h[3 * e + 1] = c * (dy - uy * ud); h[3 * e + 2] = c * (dz - uz * ud);
 }
 
-// Segmented sums of K-wide rows (the backward of gathering a per-structure table by structure index): out[b, k] =
-// sum over the rows of segment b (rows perm[seg[b]] .. perm[seg[b + 1] - 1], or seg[b] .. seg[b + 1] - 1 without
-// perm) of g[row, k].  One workgroup per segment; every thread sums a fixed stride of rows, then a fixed-order tree
-// over the workgroup: deterministic, no atomics.
+// Segmented sums of 3x3 rows (the backward of gathering a per-structure table by structure index): out[b] = sum over
+// the rows of segment b (rows perm[lo] .. perm[hi - 1], or lo .. hi - 1 without perm; lo = seg[b], or rowptr[seg[b]])
+// of g[row] (9 wide) or, with ``left``, of the outer product left[row] x g[row] (3 wide each: formed here, a [rows, 9]
+// product written and read back was four launches).  ``slices`` workgroups per segment, each writing its own out row;
+// every thread sums a fixed stride of rows, then a fixed-order tree: deterministic, no atomics.  ``gleft`` gets
+// g + sym g of each row.  With ``cell`` (one slice) the workgroup ends with dL/dsym = sum + cell^T G, G the sum of the
+// ``nparts`` rows of ``parts``, and writes its symmetric part, dL/ddisplacement.
+// Bound by the serial chain of a thread's rows: 1,024 threads per segment, 5.5 rows each on a 160-atom structure.
 #define SEG_K 9
-extern "C" __global__ __launch_bounds__(BLOCK) void geom_segsum(const float* __restrict__ g,
-    const int* __restrict__ perm, const long long* __restrict__ seg, float* __restrict__ out, int B) {
-  const int b = blockIdx.x;
+#define SEG_BLOCK 1024
+extern "C" __global__ __launch_bounds__(SEG_BLOCK) void geom_segsum(const float* __restrict__ g,
+    const int* __restrict__ perm, const long long* __restrict__ seg, float* __restrict__ out, int B,
+    const float* __restrict__ left, const int* __restrict__ rowptr, int n, int slices,
+    const float* __restrict__ cell, const float* __restrict__ parts, int nparts, const float* __restrict__ disp,
+    float* __restrict__ gleft) {
+  const int b = blockIdx.x / slices, sl = blockIdx.x - b * slices;
   if (b >= B) return;
-  const long long lo = seg[b], hi = seg[b + 1];
-  float acc[SEG_K];
+  long long lo = seg[b], hi = seg[b + 1];
+  if (left) {                      // (segments of atoms: never past the n rows there are)
+    lo = lo < 0 ? 0 : lo > n ? n : lo;
+    hi = hi < 0 ? 0 : hi > n ? n : hi;
+    if (rowptr) { lo = rowptr[lo]; hi = rowptr[hi]; }
+  }
+  const long long per = (hi - lo + slices - 1) / slices;
+  const long long from = lo + sl * per, to = from + per < hi ? from + per : hi;
+  float acc[SEG_K], sym[SEG_K];
   for (int k = 0; k < SEG_K; ++k) acc[k] = 0.f;
-  for (long long r = lo + threadIdx.x; r < hi; r += BLOCK) {
+  if (gleft) {
+    const float* d = disp + (long long)b * 9;
+    for (int k = 0; k < 9; ++k) sym[k] = 0.5f * (d[k] + d[(k % 3) * 3 + k / 3]);
+  }
+#pragma unroll 4
+  for (long long r = from + threadIdx.x; r < to; r += SEG_BLOCK) {
     const long long row = perm ? (long long)perm[r] : r;
-    for (int k = 0; k < SEG_K; ++k) acc[k] += g[row * SEG_K + k];
+    if (left) {
+      const float a0 = left[3 * row], a1 = left[3 * row + 1], a2 = left[3 * row + 2];
+      const float g0 = g[3 * row], g1 = g[3 * row + 1], g2 = g[3 * row + 2];
+      acc[0] += a0 * g0; acc[1] += a0 * g1; acc[2] += a0 * g2;
+      acc[3] += a1 * g0; acc[4] += a1 * g1; acc[5] += a1 * g2;
+      acc[6] += a2 * g0; acc[7] += a2 * g1; acc[8] += a2 * g2;
+      if (gleft) {
+        gleft[3 * row] = g0 + (sym[0] * g0 + sym[1] * g1 + sym[2] * g2);
+        gleft[3 * row + 1] = g1 + (sym[3] * g0 + sym[4] * g1 + sym[5] * g2);
+        gleft[3 * row + 2] = g2 + (sym[6] * g0 + sym[7] * g1 + sym[8] * g2);
+      }
+    } else {
+      for (int k = 0; k < SEG_K; ++k) acc[k] += g[row * SEG_K + k];
+    }
   }
-  __shared__ float red[SEG_K][BLOCK];
-  for (int k = 0; k < SEG_K; ++k) red[k][threadIdx.x] = acc[k];
+  __shared__ float red[SEG_BLOCK / 64][SEG_K], tot[SEG_K];
+  for (int k = 0; k < SEG_K; ++k) {
+    const float v = geom_wave_sum(acc[k]);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6][k] = v;
+  }
   __syncthreads();
-  for (int w = BLOCK / 2; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w)
-      for (int k = 0; k < SEG_K; ++k) red[k][threadIdx.x] += red[k][threadIdx.x + w];
-    __syncthreads();
+  if (threadIdx.x < SEG_K) {
+    float v = 0.f;
+    for (int w = 0; w < SEG_BLOCK / 64; ++w) v += red[w][threadIdx.x];
+    if (cell) {
+      const int i = threadIdx.x / 3, k = threadIdx.x % 3;
+      for (int a = 0; a < 3; ++a) {
+        float G = 0.f;
+        for (int p = 0; p < nparts; ++p) G += parts[((long long)b * nparts + p) * SEG_K + 3 * a + k];
+        v += cell[(long long)b * 9 + 3 * a + i] * G;
+      }
+    }
+    tot[threadIdx.x] = v;
   }
-  if (threadIdx.x < SEG_K) out[(long long)b * SEG_K + threadIdx.x] = red[threadIdx.x][0];
+  __syncthreads();
+  if (threadIdx.x < SEG_K) {
+    const int k = threadIdx.x;
+    out[(long long)blockIdx.x * SEG_K + k] = cell ? 0.5f * (tot[k] + tot[(k % 3) * 3 + k / 3]) : tot[k];
+  }
+}
+
+// MACE's get_symmetric_displacement in one pass: sym = (D + D^T) / 2 per structure, positions + positions sym[batch]
+// and shifts = unit_shifts (cell + cell sym)[batch[sender]].  Thread i does atom i and edge i.  A structure index
+// outside 0 .. B - 1 (or -B .. -1, counted from the end) gives NaN.  Launch-bound: 14 launches of PyTorch before.
+extern "C" __global__ __launch_bounds__(BLOCK) void geom_strain(const float* __restrict__ pos,
+    const float* __restrict__ unit, const float* __restrict__ cell, const float* __restrict__ disp,
+    const long long* __restrict__ batch, const int* __restrict__ send, float* __restrict__ opos,
+    float* __restrict__ osh, int N, long long E, int B) {
+  const long long i = (long long)blockIdx.x * BLOCK + threadIdx.x;
+#pragma unroll
+  for (int edge = 0; edge < 2; ++edge) {
+    if (i >= (edge ? E : (long long)N)) continue;
+    long long b = batch[edge ? (long long)send[i] : i];
+    if (b < 0) b += B;
+    const bool ok = b >= 0 && b < B;
+    b = ok ? b : 0;
+    const float* d = disp + b * 9;
+    float sym[9];
+    for (int k = 0; k < 9; ++k) sym[k] = 0.5f * (d[k] + d[(k % 3) * 3 + k / 3]);
+    const float* v = (edge ? unit : pos) + 3 * i;
+    const float v0 = v[0], v1 = v[1], v2 = v[2];
+    float* o = (edge ? osh : opos) + 3 * i;
+    const float* c = cell + b * 9;
+    float r[3];
+    for (int k = 0; k < 3; ++k) {
+      float m[3];
+      for (int a = 0; a < 3; ++a)
+        m[a] = edge ? c[3 * a + k] + (c[3 * a] * sym[k] + c[3 * a + 1] * sym[3 + k] + c[3 * a + 2] * sym[6 + k])
+                    : sym[3 * a + k];
+      r[k] = v0 * m[0] + v1 * m[1] + v2 * m[2];
+      if (!edge) r[k] = (k == 0 ? v0 : k == 1 ? v1 : v2) + r[k];
+    }
+    for (int k = 0; k < 3; ++k) o[k] = ok ? r[k] : __builtin_nanf("");
+  }
+}
+
+// Determinants of 3x3 matrices (a structure's volume), expanded in float64 and rounded once: torch.linalg.det is an LU
+// factorisation and eleven small kernels behind it.
+extern "C" __global__ __launch_bounds__(BLOCK) void geom_det(const float* __restrict__ a, float* __restrict__ out,
+    int B) {
+  const int b = blockIdx.x * BLOCK + threadIdx.x;
+  if (b >= B) return;
+  double m[9];
+  for (int k = 0; k < 9; ++k) m[k] = a[(long long)b * 9 + k];
+  out[b] = (float)(m[0] * (m[4] * m[8] - m[5] * m[7]) - m[1] * (m[3] * m[8] - m[5] * m[6])
+                   + m[2] * (m[3] * m[7] - m[4] * m[6]));
 }
 
 // The same for one column (MACE's per-structure energy sums): out[b] = sum of g[seg[b]] .. g[seg[b + 1] - 1].
@@ -189,7 +291,9 @@ def _module(device):
             _modules[key] = _native.Module(code, {_native.MH_GEOM_FWD: ('geom_fwd', BLOCK, BLOCK),
                                                   _native.MH_GEOM_BWD: ('geom_bwd', BLOCK, BLOCK // 64),
                                                   _native.MH_GEOM_JVP: ('geom_jvp', BLOCK, BLOCK),
-                                                  _native.MH_GEOM_SEGSUM: ('geom_segsum', BLOCK, 1),
+                                                  _native.MH_GEOM_SEGSUM: ('geom_segsum', SEG_BLOCK, 1),
+                                                  _native.MH_GEOM_STRAIN: ('geom_strain', BLOCK, BLOCK),
+                                                  _native.MH_GEOM_DET: ('geom_det', BLOCK, BLOCK),
                                                   _native.MH_GEOM_SEGSUM1: ('geom_segsum1', BLOCK, 1)})
     return _modules[key]
 
@@ -396,6 +500,47 @@ def structure_sum(src, batch, ptr):
     return _StructureSum.apply(src, batch, ptr.to(torch.int64).contiguous())
 
 
+class _StrainFn(torch.autograd.Function):
+    """positions and shifts of ``symmetric_displacement`` as a function of the displacement and the positions: one
+    launch, and two segmented sums (edges, then atoms) in the backward."""
+
+    @staticmethod
+    def forward(ctx, displacement, positions, unit_shifts, cell, batch, ptr, gr):
+        D, p, u, c = (t.contiguous() for t in (displacement, positions, unit_shifts, cell))
+        N, E, B = p.shape[0], u.shape[0], D.shape[0]
+        opos, osh = torch.empty_like(p), torch.empty_like(u)
+        P = _native.ptr
+        _native.launch('geom_strain', _native.load().mh_geom_strain, _module(p.device).handle, P(p), P(u), P(c), P(D),
+                       P(batch), P(gr.send), P(opos), P(osh), N, E, B, _native.stream_of(p))
+        ctx.save_for_backward(D, p, u, c, ptr)
+        ctx.gr = gr
+        return opos, osh
+
+    @staticmethod
+    def backward(ctx, gp, gs):
+        if torch.is_grad_enabled():          # only true under create_graph=True
+            raise RuntimeError(_DOUBLE_BACKWARD)
+        D, p, u, c, ptr = ctx.saved_tensors
+        N, E, B = p.shape[0], u.shape[0], D.shape[0]
+        gp, gs = gp.contiguous(), gs.contiguous()
+        rp_s, ei_s = ctx.gr.by_send()
+        slices = min(max(-(-E // (max(B, 1) * SLICE_ROWS)), 1), MAX_SLICES)
+        parts = torch.empty(B * slices, 9, device=p.device, dtype=torch.float32)
+        gD, gpos = torch.empty_like(D), torch.empty_like(p)
+        if E == 0:
+            parts.zero_()
+        if N == 0:
+            return gD.zero_(), gpos, None, None, None, None, None
+        m, lib, P, st = _module(p.device).handle, _native.load(), _native.ptr, _native.stream_of(p)
+        # dL/dcell' = sum of unit_shift x g_shift over the structure's edges, then dL/dsym over its atoms
+        if E:
+            _native.launch('geom_segsum', lib.mh_geom_strain_sum, m, P(u), P(gs), P(ei_s), P(ptr), P(rp_s), N,
+                           P(parts), slices, None, None, 0, None, None, B, st)
+        _native.launch('geom_segsum', lib.mh_geom_strain_sum, m, P(p), P(gp), None, P(ptr), None, N, P(gD), 1, P(c),
+                       P(parts), slices, P(D), P(gpos), B, st)
+        return gD, gpos, None, None, None, None, None
+
+
 def symmetric_displacement(positions, unit_shifts, cell, edge_index, num_graphs, batch, ptr):
     """MACE's ``get_symmetric_displacement`` (positions and shifts under a symmetric strain of each structure's cell,
     for the virials and the stress) with its two per-structure gathers, sym[batch] over the atoms and
@@ -406,6 +551,12 @@ def symmetric_displacement(positions, unit_shifts, cell, edge_index, num_graphs,
     n = positions.shape[0]
     displacement = torch.zeros((num_graphs, 3, 3), dtype=positions.dtype, device=positions.device)
     displacement.requires_grad_(True)
+    if _ACTIVE.get() is True and batch.dtype == torch.int64 and not (cell.requires_grad or unit_shifts.requires_grad):
+        # a first-order call with constant cell and unit shifts (a force loss differentiates the strain twice)
+        positions, shifts = _StrainFn.apply(displacement, positions, unit_shifts, cell.view(-1, 3, 3),
+                                            batch.contiguous(), ptr.to(torch.int64).contiguous(),
+                                            _conv.graph_for(edge_index, n))
+        return positions, shifts, displacement
     sym = 0.5 * (displacement + displacement.transpose(-1, -2))
     seg_atoms = ptr.to(torch.int64).contiguous()
     # row vector times a 3x3 matrix per row, as a broadcast product and a sum over three terms: the einsum / matmul
@@ -458,6 +609,54 @@ def _wrap_displacement(orig):
         return orig(positions, unit_shifts, cell, edge_index, num_graphs, batch)
     get_symmetric_displacement._mh_original = orig
     return get_symmetric_displacement
+
+
+def _det3(a):
+    out = torch.empty(a.shape[0], device=a.device, dtype=torch.float32)
+    _native.launch('geom_det', _native.load().mh_geom_det, _module(a.device).handle, _native.ptr(a), _native.ptr(out),
+                   a.shape[0], _native.stream_of(a))
+    return out
+
+
+class _Cell(torch.Tensor):
+    """The cells handed to MACE's ``get_outputs``: a view of the caller's tensor whose determinants (the volumes that
+    the stress is divided by) are one kernel.  A reshaped view stays one; anything else gives plain tensors."""
+
+    @classmethod
+    def __torch_function__(cls, func, types, args=(), kwargs=None):
+        kwargs = kwargs or {}
+        with torch._C.DisableTorchFunctionSubclass():
+            if func in _DETS and len(args) == 1 and not kwargs and args[0].dim() == 3 and args[0].shape[1:] == (3, 3):
+                return _det3(args[0].contiguous())
+            out = func(*args, **kwargs)
+            return out.as_subclass(cls) if func in _VIEWS and args[0].__class__ is cls else out
+
+
+_DETS = {torch.linalg.det, torch.det, torch.Tensor.det}
+_VIEWS = {torch.Tensor.view, torch.Tensor.reshape, torch.reshape}
+
+
+def _wrap_outputs(orig):
+    try:
+        names = list(inspect.signature(orig).parameters)
+    except (TypeError, ValueError):
+        names = []
+    at = names.index('cell') if 'cell' in names else -1
+
+    @functools.wraps(orig)
+    def get_outputs(*args, **kwargs):
+        if _ACTIVE.get() and at >= 0:
+            cell = args[at] if at < len(args) else kwargs.get('cell')
+            if (type(cell) is torch.Tensor and cell.is_cuda and cell.dtype == torch.float32 and cell.numel() > 0
+                    and not cell.requires_grad):
+                c = cell.as_subclass(_Cell)
+                if at < len(args):
+                    args = args[:at] + (c,) + args[at + 1:]
+                else:
+                    kwargs = dict(kwargs, cell=c)
+        return orig(*args, **kwargs)
+    get_outputs._mh_original = orig
+    return get_outputs
 
 
 def _wrap_scatter(orig):
@@ -527,6 +726,9 @@ def install(model):
     disp = getattr(mod, DISPLACEMENT, None)
     if callable(disp) and not hasattr(disp, '_mh_original'):
         setattr(mod, DISPLACEMENT, _wrap_displacement(disp))
+    outs = getattr(mod, OUTPUTS, None)
+    if callable(outs) and not hasattr(outs, '_mh_original'):
+        setattr(mod, OUTPUTS, _wrap_outputs(outs))
     sc = getattr(mod, SCATTER, None)
     if callable(sc) and not hasattr(sc, '_mh_original'):
         setattr(mod, SCATTER, _wrap_scatter(sc))
