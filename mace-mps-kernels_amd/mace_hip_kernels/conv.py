@@ -178,18 +178,33 @@ extern "C" __global__ __launch_bounds__(256) void csr_fill(int* __restrict__ cnt
   if (i == 0 && blockIdx.y == 0) bad[0] = 0;
 }
 
+// A wave's lanes in runs of equal consecutive keys (every lane of the wave calls this): the first lane of this lane's
+// run and, for that lane, the run's length.  Edge lists come sorted by one endpoint and padded with self-loops of one
+// atom, so a counter otherwise takes the wave's 64 atomics one after another.
+__device__ __forceinline__ int csr_run(int k, int& len) {
+  const int lane = threadIdx.x & 63, before = __shfl_up(k, 1, 64);
+  const unsigned long long lead = __ballot(lane == 0 || before != k);
+  const unsigned long long after = lane == 63 ? 0ull : lead >> (lane + 1);
+  len = after ? __ffsll(after) : 64 - lane;
+  return 63 - __clzll(lead & (~0ull >> (63 - lane)));
+}
+
 extern "C" __global__ __launch_bounds__(256) void csr_count(const long long* __restrict__ index, int* __restrict__ keys,
     int* __restrict__ cnt, int* __restrict__ bad, long long E, int n) {
   const long long e = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (e >= E) return;
   const long long r = blockIdx.y;
-  long long k = index[r * E + e];
-  if (k < 0 || k >= n) {                  // flagged for the caller; clamped so that nothing reads out of range
-    atomicOr(bad, 1);
-    k = k < 0 ? 0 : n - 1;
+  long long k = -1;                       // a lane past the list: a run of its own
+  if (e < E) {
+    k = index[r * E + e];
+    if (k < 0 || k >= n) {                // flagged for the caller; clamped so that nothing reads out of range
+      atomicOr(bad, 1);
+      k = k < 0 ? 0 : n - 1;
+    }
+    keys[r * E + e] = (int)k;
   }
-  keys[r * E + e] = (int)k;
-  atomicAdd(&cnt[r * (n + 1) + k], 1);
+  int len;
+  const int first = csr_run((int)k, len);
+  if (e < E && first == (int)(threadIdx.x & 63)) atomicAdd(&cnt[r * (n + 1) + k], len);
 }
 
 extern "C" __global__ __launch_bounds__(1024) void csr_scan(const int* __restrict__ cnt, int* __restrict__ rowptr,
@@ -213,10 +228,13 @@ extern "C" __global__ __launch_bounds__(1024) void csr_scan(const int* __restric
 extern "C" __global__ __launch_bounds__(256) void csr_scatter(const int* __restrict__ keys, int* __restrict__ cursor,
     int* __restrict__ tmp, long long E, int n) {
   const long long e = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (e >= E) return;
   const long long r = blockIdx.y;
-  const int pos = atomicAdd(&cursor[r * (n + 1) + keys[r * E + e]], 1);
-  tmp[r * E + pos] = (int)e;
+  const int k = e < E ? keys[r * E + e] : -1, lane = threadIdx.x & 63;
+  int len, pos = 0;
+  const int first = csr_run(k, len);
+  if (e < E && first == lane) pos = atomicAdd(&cursor[r * (n + 1) + k], len);
+  pos = __shfl(pos, first, 64) + lane - first;
+  if (e < E) tmp[r * E + pos] = (int)e;
 }
 
 extern "C" __global__ __launch_bounds__(256) void csr_rank(const int* __restrict__ keys, const int* __restrict__ rowptr,
