@@ -119,7 +119,8 @@ enum mh_kernel_kind {
     MH_CONV_BWD_T = 80,  /* convolution backward to the lengths: gY, dL/dlength, dX messages, no dL/dW         */
     MH_GEOM_STRAIN = 81, /* stress displacement: strained positions and shifts                                 */
     MH_GEOM_DET = 82,    /* determinants of 3x3 matrices                                                       */
-    MH_NUM_KINDS = 83
+    MH_MLP_BWD_W = 83,   /* radial MLP backward, column slices: their sum walked back through the hidden layers */
+    MH_NUM_KINDS = 84
 };
 
 /* flags of mh_conv_bwd */
@@ -517,6 +518,13 @@ int mh_mlp_fwd_ws(mh_module* m, const float* ef, const float* WhT, const uint16_
                   int64_t E, const int32_t* rows, const int32_t* count, int32_t ncb, void* stream);
 int mh_mlp_bwd_rows(mh_module* m, const float* ef, const float* Wh, const uint16_t* Wl, const float* gW0, float* gef,
                     int64_t E, const int32_t* rows, const int32_t* count, void* stream);
+/* mh_mlp_bwd for few edges: the output columns in `slices` shares (at most one per chunk of 32 columns, none empty: the
+ * share is ceil(chunks / slices)), whose partial dL/dh go to part [slices][E][last hidden width], then their sum walked
+ * back (MH_MLP_BWD with `slices` rows of workgroups and MH_MLP_BWD_W, bound with 256 threads and 64 edges).  No
+ * reference counterpart. */
+int mh_mlp_bwd_split(mh_module* m, const float* ef, const float* Wh, const uint16_t* Wl, const float* gW0, float* gef,
+                     int64_t E, float* part, int32_t slices, void* stream);
+
 /* mh_mlp_bwd_rows over the rows mh_edge_pairs shares between an edge and its exact reverse: slot i < count[0]
  * (edge e = rows[i], a row the forward computed) projects gW0[e] + gW0[partner[e]] when partner[e] >= 0 (the one
  * edge that reads e's W0 row, from mh_edge_pairs with vec), else gW0[e]; gef[e] receives the row's gradient and

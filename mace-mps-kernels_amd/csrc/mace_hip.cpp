@@ -146,7 +146,7 @@ extern "C" {
 
 const char* mh_last_error(void) { return g_err.c_str(); }
 
-int mh_version(void) { return 44; }
+int mh_version(void) { return 45; }
 
 int mh_launch_log(int enable) {
     std::lock_guard<std::mutex> lock(g_log_mu);
@@ -942,8 +942,21 @@ int mh_mlp_bwd_rows(mh_module* m, const float* ef, const float* Wh, const uint16
                     int64_t E, const int32_t* rows, const int32_t* count, void* stream) {
     if (E > 0 && (!ef || !Wh || !Wl || !gW0 || !gef)) return fail(-1, "mh_mlp_bwd: NULL operand");
     if ((rows == nullptr) != (count == nullptr)) return fail(-1, "mh_mlp_bwd_rows: rows and count go together");
-    void* args[] = {&ef, &Wh, &Wl, &gW0, &gef, &E, &rows, &count};
+    float* part = nullptr;
+    void* args[] = {&ef, &Wh, &Wl, &gW0, &gef, &E, &rows, &count, &part};
     return launch(m, MH_MLP_BWD, E, args, stream, "mh_mlp_bwd");
+}
+
+int mh_mlp_bwd_split(mh_module* m, const float* ef, const float* Wh, const uint16_t* Wl, const float* gW0, float* gef,
+                     int64_t E, float* part, int32_t slices, void* stream) {
+    if (E > 0 && (!ef || !Wh || !Wl || !gW0 || !gef || !part)) return fail(-1, "mh_mlp_bwd_split: NULL operand");
+    if (slices < 2 || slices > 0xffff) return fail(-1, "mh_mlp_bwd_split: slices out of range");
+    const int32_t* rows = nullptr;
+    const int32_t* count = nullptr;
+    void* args[] = {&ef, &Wh, &Wl, &gW0, &gef, &E, &rows, &count, &part};
+    if (int rc = launch(m, MH_MLP_BWD, E, args, stream, "mh_mlp_bwd_split", slices)) return rc;
+    void* walk[] = {&ef, &Wh, &part, &slices, &gef, &E};
+    return launch(m, MH_MLP_BWD_W, E, walk, stream, "mh_mlp_bwd_split");
 }
 
 int mh_mlp_bwd_pairs(mh_module* m, const float* ef, const float* Wh, const uint16_t* Wl, const float* gW0,

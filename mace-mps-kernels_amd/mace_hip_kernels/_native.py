@@ -28,9 +28,9 @@ MH_CONV_FWD, MH_CONV_BWD, MH_CONV_BWD_WY, MH_SC_FWD, MH_SC_BWD, MH_CONV_BWD_R, M
     MH_NL_FILL, MH_SPECIES_ORDER, MH_MLP_JVP, MH_MLP_BWD2, MH_GEOM_SEGSUM, MH_NL_BASES, MH_EDGE_COUNT, \
     MH_EDGE_PLACE, MH_GEOM_SEGSUM1, MH_EDGE_PAIR, MH_CONV_FWD_CR, MH_MLP_H3, MH_MLP_OUT, MH_EDGE_FWD, \
     MH_EDGE_BWD, MH_MLP_BWD_P, MH_LIN_BWD_SUM, MH_MLP_H3T, MH_CONV_BWD_T, \
-    MH_GEOM_STRAIN, MH_GEOM_DET = range(83)
+    MH_GEOM_STRAIN, MH_GEOM_DET, MH_MLP_BWD_W = range(84)
 MH_WANT_GX, MH_WANT_GWY, MH_CUT_MASKED, MH_CUT_NOZERO = 1, 2, 4, 8
-ABI_VERSION = 44
+ABI_VERSION = 45
 
 # hipcc/hipRTC options for every generated layer: gfx950 code, -O3, and packed-FP32 instructions disabled.
 ARCH = os.environ.get('MACE_HIP_ARCH', 'gfx950')
@@ -73,6 +73,7 @@ _SIGS = {
     'mh_mlp_fwd_rows': (ctypes.c_int, [_P] * 5 + [ctypes.c_int64, _P, _P, _P]),
     'mh_mlp_fwd_ws': (ctypes.c_int, [_P] * 6 + [ctypes.c_int64, _P, _P, ctypes.c_int32, _P]),
     'mh_mlp_bwd_rows': (ctypes.c_int, [_P] * 6 + [ctypes.c_int64, _P, _P, _P]),
+    'mh_mlp_bwd_split': (ctypes.c_int, [_P] * 6 + [ctypes.c_int64, _P, _I, _P]),
     'mh_mlp_bwd_pairs': (ctypes.c_int, [_P] * 6 + [ctypes.c_int64, _P, _P, _P, _P]),
     'mh_edge_compact_work_size': (ctypes.c_size_t, [ctypes.c_int64]),
     'mh_geom_segsum1': (ctypes.c_int, [_P, _P, _P, _P, _I, _P]),

@@ -71,6 +71,16 @@ WAVES_BWD = 3
 # more waves: config 2, layer 2 / layer 1 in the E+F call, 4 waves 143.6 / 72.6 us, 6 waves 157.6 / 84.2, 8 waves
 # 172.1 / 84.0.
 WG_WAVES_BWD = 4
+# Few edges leave most compute units idle while each workgroup walks every output column in turn (one L2 round trip per
+# chunk of 32): the columns are then split over blockIdx.y, at least SPLIT_CHUNKS chunks per workgroup and about
+# SPLIT_BLOCKS workgroups in all (one per compute unit), into partial dL/dh rows that mlp_bwd_w sums and walks back.
+# Measured (us, unsplit / 2 / 5 / 10 slices): 1280 columns, 1,500 edges 30 / - / - / 18, 2,700 30 / - / 20 / 22, 5,462
+# 32 / 25 / 23 / 28, 9,000 34 / - / 26 (3) / 30 (7), 16,000 35 / 32 / - / -, 40,000 65 unsplit.  512 columns (unsplit /
+# 2 / 4 slices): 1,500 17.6 / - / 14.8, 2,700 17.6 / - / 15.9, 5,462 17.4 / 16.9 / 18.4, 9,000 17.5 / - / 20 (3): fewer
+# than SPLIT_WIDE chunks save less than the second launch costs once the workgroups no longer run at the same time.
+SPLIT_CHUNKS = 4
+SPLIT_BLOCKS = 256
+SPLIT_WIDE = 32
 # The forward as two kernels (mh_mlp_fwd_ws): the hidden layers of the listed rows into an [E, HL] scratch (mlp_h3),
 # then the output layer weight-stationary (mlp_out): a persistent grid whose waves each keep one block of WS_COLS
 # output columns of the split output layer in registers and walk the 16-edge tiles of their XCD's share, four waves
@@ -565,7 +575,8 @@ def _source(spec, second):
         """The backward (``dual``: the Hessian-vector product along ev; ``paired``: ``mlp_bwdp``, the row list's
         slot i < count[0] (edge e = rows[i]) projects the sum of e's dL/dW0 row and that of partner[e] when
         partner[e] >= 0, the edge that reads e's W0 row; the partner's own slot lies past count[0] and gets a zero
-        dL/d(edge features) row like every other uncomputed slot)."""
+        dL/d(edge features) row like every other uncomputed slot).  ``mlp_bwd`` launched with blockIdx.y slices does a
+        share of the output columns each and stores its partial dL/dh to ``part`` [slices][E][HL] (``mlp_bwd_w``)."""
         # dL/dh_last = gW Wl^T first: K = the output columns, one bf16 step of 32 per chunk (lane group q: columns
         # 8 q .. 8 q + 7, two float4 loads of gW split into three bf16 parts); chunks of Wl [HL][CH] as bf16 rows of
         # CH + BPAD.  Then the hidden layers recomputed from the natural-layout fp32 weights and walked back.
@@ -581,7 +592,9 @@ def _source(spec, second):
         B = head(name, 'const float* __restrict__ ef, ' + ('const float* __restrict__ ev, ' if dual else '') +
                  'const float* __restrict__ Wh, const unsigned short* __restrict__ Wl, const float* __restrict__ gW, '
                  'float* __restrict__ gef, long long E', lds_bwd, nb, waves=wg, indexed=not dual,
-                 wpe=None if dual else WAVES_BWD, extra=', const int* __restrict__ partner' if paired else '')
+                 wpe=None if dual else WAVES_BWD,
+                 extra=', const int* __restrict__ partner' if paired else '' if dual else ', float* __restrict__ part')
+        split = not (dual or paired)
         if not dual:
             B += skip_block(nb, zero_rows=True, waves=wg)
         if paired:
@@ -593,7 +606,13 @@ def _source(spec, second):
         for b in range(nb):
             B += [f'  mh_f4 dh{b}[{TL}][{ncb}];'] + [f'  dh{b}[{o}][{j}] = mh_f4{{0.f, 0.f, 0.f, 0.f}};'
                                                     for o in range(TL) for j in range(ncb)]
-        ld0, npre = chunk_io('Wl', 0, CH, RSB, HL, '  ', nthreads=nt)
+        first, last = '0', str(NCHK)
+        if split:                        # this slice's chunks ch0 .. ch1 - 1 (the launcher leaves no slice empty)
+            B += [f'  const int per = ({NCHK} + (int)gridDim.y - 1) / (int)gridDim.y, ch0 = (int)blockIdx.y * per;',
+                  f'  const int ch1 = min(ch0 + per, {NCHK});']
+            first, last = 'ch0', 'ch1'
+        nx0 = f'(size_t)ch0 * {NSPLIT * HL * CH}' if split else 0
+        ld0, npre = chunk_io('Wl', nx0, CH, RSB, HL, '  ', nthreads=nt)
         B += [f'  mh_u4 {", ".join(f"pre{i}" for i in range(npre))};'] + ld0
         # columns past NW (the zero-padded tail of the last chunk) read a valid column and are zeroed
         gcol = (lambda c: f'min({c} + 8 * q, {NW - 8})') if TAIL else (lambda c: f'{c} + 8 * q')
@@ -614,7 +633,9 @@ def _source(spec, second):
         # dL/dW0 of chunk ch + d sits in g{d}_* (d = 0 .. dist - 1) while chunk ch is multiplied
         for b in range(nb):
             for d in range(dist):
-                if paired:
+                if split:
+                    B += gload(f'g{d}', f'min(ch0 + {d}, ch1 - 1) * {CH}', b, '  mh_f4 ')
+                elif paired:
                     B += gload(f'gi{d}', str(min(d, NCHK - 1) * CH), b, '  mh_f4 ')
                     B += gload(f'gi{d}p', str(min(d, NCHK - 1) * CH), b, '  mh_f4 ', row='prc')
                     B += fold(f'g{d}', f'gi{d}', b, '  mh_f4 ')
@@ -622,13 +643,13 @@ def _source(spec, second):
                     B += gload(f'g{d}', str(min(d, NCHK - 1) * CH), b, '  mh_f4 ')
         st0, _ = chunk_io('Wl', 0, CH, RSB, HL, '  ', store_base='0', nthreads=nt)
         B += st0 + ['  __syncthreads();']
-        B += [f'  for (int ch = 0; ch < {NCHK}; ++ch) {{',
-              f'    const int base = (ch & 1) * {Lo["chunk_bwd"]}, nbase = {Lo["chunk_bwd"]} - base;',
-              f'    const int nc = min(ch + 1, {NCHK - 1});',
+        B += [f'  for (int ch = {first}; ch < {last}; ++ch) {{',
+              f'    const int base = ({"(ch - ch0)" if split else "ch"} & 1) * {Lo["chunk_bwd"]}, nbase = {Lo["chunk_bwd"]} - base;',
+              f'    const int nc = min(ch + 1, {last} - 1);',
               f'    const size_t nx = (size_t)nc * {NSPLIT * HL * CH};']
         ldn, _ = chunk_io('Wl', 'nx', CH, RSB, HL, '    ', nthreads=nt)
         B += ldn
-        B += [f'    const int gc = min(ch + {dist}, {NCHK - 1}) * {CH};']
+        B += [f'    const int gc = min(ch + {dist}, {last} - 1) * {CH};']
         for b in range(nb):
             B += gload('gn', 'gc', b, '    const mh_f4 ')
             if paired:
@@ -666,6 +687,14 @@ def _source(spec, second):
         for b in range(nb):
             B += [f'  mh_f4 dhs_{b}[{TL}];'] + [f'  dhs_{b}[{o}] = ' + ' + '.join(f'dh{b}[{o}][{j}]' for j in range(ncb)) + ';'
                                                for o in range(TL)]
+        if split:
+            B += ['  if (gridDim.y > 1) {']
+            for b in range(nb):
+                B += [f'    if (live{b}) {{',
+                      f'      float* __restrict__ pr = part + ((long long)blockIdx.y * E + ej{b}) * {HL} + 4 * q;']
+                B += [f'      *reinterpret_cast<mh_f4*>(pr + {16 * o}) = dhs_{b}[{o}];' for o in range(TL)]
+                B += ['    }']
+            B += ['    return;', '  }']
         # the hidden layers recomputed and walked back HIDDEN_TILES_BWD edge tiles at a time (each group in a scope of
         # its own, so the registers of its activations are free for the next)
         B += stage('Wh', Lo['nat_size'], nthreads=nt) + ['  __syncthreads();']
@@ -680,6 +709,20 @@ def _source(spec, second):
             B += ['  }', '  __builtin_amdgcn_sched_barrier(0);       // one group finished before the next starts']
         B += ['}', '']
         return B
+
+    def walk_kernel(name):
+        """mlp_bwd_w: the hidden half of mlp_bwd for a split launch: dL/dh_last of edge e = the sum over the slices of
+        part[slice][e], in order, walked back to dL/d(edge features)."""
+        grp = range(1)
+        H = head(name, 'const float* __restrict__ ef, const float* __restrict__ Wh, const float* __restrict__ part, '
+                 'int slices, float* __restrict__ gef, long long E', Lo['nat_size'], 1)
+        H += xin(grp) + stage('Wh', Lo['nat_size'])
+        H += [f'  mh_f4 dhs_0[{TL}];'] + [f'  dhs_0[{o}] = mh_f4{{0.f, 0.f, 0.f, 0.f}};' for o in range(TL)]
+        H += ['#pragma unroll 2', '  for (int s = 0; s < slices; ++s) {',
+              f'    const float* __restrict__ pr = part + ((long long)s * E + ejc0) * {HL} + 4 * q;']
+        H += [f'    dhs_0[{o}] += *reinterpret_cast<const mh_f4*>(pr + {16 * o});' for o in range(TL)]
+        H += ['  }', '  __syncthreads();'] + hidden_fwd(False, False, grp) + walk_back(grp, 'dhs_')
+        return H + ['}', '']
 
     def hidden_only():
         """mlp_hid / mlp_hidb, the fused convolution's MLP kernels."""
@@ -923,7 +966,7 @@ def _source(spec, second):
         L += fwd_kernel(spec.kname('mlp_jvp'), True) + bwd_kernel(spec.kname('mlp_bwd2'), True)
     else:
         L += fwd_kernel(spec.kname('mlp_fwd'), False) + bwd_kernel(spec.kname('mlp_bwd'), False)
-        L += bwd_kernel(spec.kname('mlp_bwdp'), False, paired=True)
+        L += bwd_kernel(spec.kname('mlp_bwdp'), False, paired=True) + walk_kernel(spec.kname('mlp_bwd_w'))
         hidden_only()
         L += h3_kernel(spec.kname('mlp_h3')) + out_kernel(spec.kname('mlp_out'))
         L += h3t_kernel(spec.kname('mlp_bwdp_h'))
@@ -978,6 +1021,15 @@ _DOUBLE_BACKWARD = ('mace_hip_kernels: double backward (create_graph=True, e.g. 
                     'patch_model(model, double_backward=True)')
 
 
+def bwd_slices(n_out, E):
+    """Column slices of the backward over E edges and n_out output columns (1: a single launch)."""
+    blocks, chunks = -(-E // (16 * NB_BWD * WG_WAVES_BWD)), -(-n_out // CH_BWD)
+    blocks = max(blocks, 1)
+    want = SPLIT_BLOCKS // blocks if chunks < SPLIT_WIDE else -(-SPLIT_BLOCKS // blocks)
+    want = min(want, chunks // SPLIT_CHUNKS)
+    return 1 if want < 2 else -(-chunks // -(-chunks // want))
+
+
 def _mlp_bwd(op, ef, g, rows=None, count=None):
     """dL/d(edge features) [E, n_basis] from dL/dW0 (contiguous 2-D operands).  With a row list (``rows``,
     ``count`` from ``conv.support_rows``) only the first count[0] listed edges are computed; the others get zero rows
@@ -985,6 +1037,13 @@ def _mlp_bwd(op, ef, g, rows=None, count=None):
     gx = torch.empty_like(ef)
     P = _native.ptr
     op.bwd_paired = False
+    E = ef.shape[0]
+    slices = bwd_slices(op.spec.hs[-1], E) if rows is None else 1
+    if slices > 1:
+        part = torch.empty(slices, E, op.spec.hs[-2], device=ef.device, dtype=torch.float32)
+        _native.launch(f'mlp_bwd[{op.tag}]', _native.load().mh_mlp_bwd_split, op.module.handle, P(ef), P(op.Wh),
+                       P(op.Wl), P(g), P(gx), E, P(part), slices, _native.stream_of(ef))
+        return gx
     _native.launch(f'mlp_bwd[{op.tag}]', _native.load().mh_mlp_bwd_rows, op.module.handle, P(ef), P(op.Wh), P(op.Wl),
                    P(g), P(gx), ef.shape[0], P(rows), P(count), _native.stream_of(ef))
     return gx
@@ -1125,6 +1184,7 @@ class HipRadialMLP(torch.nn.Module):
                 _native.MH_MLP_H3: (self.spec.kname('mlp_h3'), BLOCK, 64),
                 _native.MH_MLP_OUT: (self.spec.kname('mlp_out'), BLOCK, 1),
                 _native.MH_MLP_H3T: (self.spec.kname('mlp_bwdp_h'), BLOCK, 64),
+                _native.MH_MLP_BWD_W: (self.spec.kname('mlp_bwd_w'), BLOCK, 64),
             })
         self.ncb = -(-self.spec.hs[-1] // WS_COLS)
         pw = packed_weights(self.spec)
