@@ -518,8 +518,8 @@ int mh_mlp_fwd_ws(mh_module* m, const float* ef, const float* WhT, const uint16_
                   int64_t E, const int32_t* rows, const int32_t* count, int32_t ncb, void* stream);
 int mh_mlp_bwd_rows(mh_module* m, const float* ef, const float* Wh, const uint16_t* Wl, const float* gW0, float* gef,
                     int64_t E, const int32_t* rows, const int32_t* count, void* stream);
-/* mh_mlp_bwd for few edges: the output columns in `slices` shares (at most one per chunk of 32 columns, none empty: the
- * share is ceil(chunks / slices)), whose partial dL/dh go to part [slices][E][last hidden width], then their sum walked
+/* mh_mlp_bwd for few edges: the output columns in `slices` shares of ceil(chunks / slices) chunks of 32 columns (the last
+ * ones may be empty), whose partial dL/dh go to part [slices][E][last hidden width], then their sum walked
  * back (MH_MLP_BWD with `slices` rows of workgroups and MH_MLP_BWD_W, bound with 256 threads and 64 edges).  No
  * reference counterpart. */
 int mh_mlp_bwd_split(mh_module* m, const float* ef, const float* Wh, const uint16_t* Wl, const float* gW0, float* gef,

@@ -607,11 +607,11 @@ def _source(spec, second):
             B += [f'  mh_f4 dh{b}[{TL}][{ncb}];'] + [f'  dh{b}[{o}][{j}] = mh_f4{{0.f, 0.f, 0.f, 0.f}};'
                                                     for o in range(TL) for j in range(ncb)]
         first, last = '0', str(NCHK)
-        if split:                        # this slice's chunks ch0 .. ch1 - 1 (the launcher leaves no slice empty)
+        if split:                        # this slice's chunks ch0 .. ch1 - 1 (none past the last: a zero share)
             B += [f'  const int per = ({NCHK} + (int)gridDim.y - 1) / (int)gridDim.y, ch0 = (int)blockIdx.y * per;',
                   f'  const int ch1 = min(ch0 + per, {NCHK});']
             first, last = 'ch0', 'ch1'
-        nx0 = f'(size_t)ch0 * {NSPLIT * HL * CH}' if split else 0
+        nx0 = f'(size_t)min(ch0, {NCHK - 1}) * {NSPLIT * HL * CH}' if split else 0
         ld0, npre = chunk_io('Wl', nx0, CH, RSB, HL, '  ', nthreads=nt)
         B += [f'  mh_u4 {", ".join(f"pre{i}" for i in range(npre))};'] + ld0
         # columns past NW (the zero-padded tail of the last chunk) read a valid column and are zeroed

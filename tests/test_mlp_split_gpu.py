@@ -38,3 +38,18 @@ def test_split_backward(monkeypatch, widths, edges):
 @pytest.mark.parametrize('edges', [16385, 40000])
 def test_many_edges_are_not_split(edges):
     assert radial.bwd_slices(1280, edges) == radial.bwd_slices(512, edges) == 1
+
+
+@pytest.mark.parametrize('slices', [2, 7, 40])
+def test_any_number_of_slices(monkeypatch, slices):
+    """16 chunks of columns in 7 and 40 shares leave the last shares empty."""
+    print(f'[case] split radial backward, {slices} slices', flush=True)
+    torch.manual_seed(slices)
+    op = radial.HipRadialMLP(enn.FullyConnectedNet([8, 64, 64, 64, 512], torch.nn.functional.silu))
+    ef, g = torch.randn(130, 8, device='cuda'), torch.randn(130, 512, device='cuda')
+    monkeypatch.setattr(radial, 'bwd_slices', lambda n_out, E: 1)
+    one = radial._mlp_bwd(op, ef, g)
+    monkeypatch.setattr(radial, 'bwd_slices', lambda n_out, E: slices)
+    got = radial._mlp_bwd(op, ef, g)
+    # the same products summed in another order (as above)
+    assert (got - one).abs().max().item() <= 4e-6 * one.abs().max().item()
