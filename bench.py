@@ -141,13 +141,26 @@ def _kernel_table(met, batch, n_real_edges, summary, symbols):
                                   HipReshapeIrreps, HipSphericalHarmonics, HipSymmetricContraction)
     n = batch['positions'].shape[0]
     n_elem_used = int((batch['node_attrs'].sum(0) > 0).sum())
-    rows = {}
+    rows, lengths = {}, {}
     for m in met.modules():
         if isinstance(m, HipConvTP):
             s = m.spec
             bf, bb = s.bytes(n, n_real_edges)
             ff, fb = s.flops()
             rows[f'conv_fwd[{m.tag}]'] = (bf, ff * n_real_edges * s.mul)
+            if any('conv_bwdt' in k for k in symbols.get(f'conv_bwd[{m.tag}]', [])):
+                # the backward to the edge lengths: the rows of W0 and dW0/dr read (one per edge and its exact
+                # reverse), no dL/dW0 written
+                mlp = m.deferred_mlp()
+                last = getattr(mlp, 'last_rows', n_real_edges)
+                nrow = int(last.item()) if torch.is_tensor(last) else int(last)
+                nw = s.nins * s.mul
+                bb += 4 * (2 * nrow * nw - 2 * n_real_edges * nw)
+                fb += 2 * s.nins                                    # the product with dW0/dr
+                rows[f'mlp_out[{mlp.tag}]'] = (4 * nrow * (mlp.spec.hs[-2] + mlp.spec.hs[-1]),
+                                               2 * nrow * mlp.spec.hs[-2] * mlp.spec.hs[-1])
+                hidden = mlp.spec.flops(nrow) - 2 * nrow * mlp.spec.hs[-2] * mlp.spec.hs[-1]
+                lengths[mlp.tag] = (4 * nrow * (2 * mlp.spec.hs[0] + mlp.spec.hs[-2]), 2 * hidden)
             rows[f'conv_bwd[{m.tag}]'] = (bb, fb * n_real_edges * s.mul)
         elif isinstance(m, HipSymmetricContraction):
             s = m.spec
@@ -191,6 +204,8 @@ def _kernel_table(met, batch, n_real_edges, summary, symbols):
             _, bb = s.bytes(eb_rows)
             rows[f'mlp_fwd[{m.tag}]'] = (bf, s.flops(ef_rows))
             rows[f'mlp_bwd[{m.tag}]'] = (bb, s.flops(ef_rows if getattr(m, 'bwd_paired', False) else eb_rows))
+    # (the radial MLP's share of the backward to the lengths: the hidden layers on dual numbers)
+    rows.update({f'mlp_bwd[{tag}]': r for tag, r in lengths.items()})
     # edge geometry: positions, shifts and the edge list in, vectors and lengths out; backward: vectors, lengths and
     # their gradients plus both CSRs in, the position gradient out
     E = batch['edge_index'].shape[1]
@@ -885,8 +900,9 @@ def main():
     if os.path.exists(tf):
         with open(tf) as fh:
             tj = json.load(fh)
-        recs = [tj['kernels'][k] for k in (d.get('symbol') or '').split('+') if k in tj['kernels']]
-        if recs:
+        parts = (d.get('symbol') or '').split('+')
+        if all(k in tj['kernels'] for k in parts):
+            recs = [tj['kernels'][k] for k in parts]
             traffic, traffic_src = int(sum(r['traffic_bytes'] for r in recs)), tj['source']
     # E+F at batch 1, 4 and 16 of config 2's structures (the reference's benchmarks/bench.py batches, its
     # README.md:64): captured and eager, and the unpatched model on the same GPU, per call and per structure
