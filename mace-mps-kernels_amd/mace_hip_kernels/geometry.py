@@ -395,6 +395,9 @@ def edge_vectors_and_lengths(positions, edge_index, shifts):
     """(vectors [E, 3], lengths [E, 1]) on the GPU kernels, differentiable in positions and shifts."""
     if positions.dtype != torch.float32 or shifts.dtype != torch.float32 or not positions.is_cuda:
         raise TypeError('mace_hip_kernels: edge geometry expects float32 GPU positions and shifts')
+    if not _together(positions, edge_index, shifts):
+        raise RuntimeError(f'mace_hip_kernels: edge geometry expects edge_index and shifts on {positions.device}, got '
+                           f'{edge_index.device}, {shifts.device}')
     if positions.shape[-1] != 3 or shifts.shape != (edge_index.shape[1], 3):
         raise ValueError(f'positions [N, 3] and shifts [E, 3] expected, got {tuple(positions.shape)}, '
                          f'{tuple(shifts.shape)}')
@@ -572,17 +575,22 @@ def symmetric_displacement(positions, unit_shifts, cell, edge_index, num_graphs,
 
 
 def _supported_displacement(positions, unit_shifts, cell, edge_index, num_graphs, batch, ptr):
-    return (_supported_call(positions, edge_index, unit_shifts) and torch.is_tensor(cell) and cell.is_cuda
-            and cell.dtype == torch.float32 and cell.numel() == 9 * num_graphs and torch.is_tensor(batch)
-            and batch.is_cuda and batch.shape == (positions.shape[0],) and torch.is_tensor(ptr) and ptr.is_cuda
+    return (_supported_call(positions, edge_index, unit_shifts) and positions.shape[1] == 3
+            and _together(positions, cell, batch, ptr) and cell.dtype == torch.float32
+            and cell.numel() == 9 * num_graphs and batch.shape == (positions.shape[0],)
             and ptr.shape == (num_graphs + 1,))
 
 
+def _together(positions, *others):
+    """Whether all are tensors of the positions' GPU (the kernels take raw pointers; elsewhere MACE's own expressions
+    report the device that differs)."""
+    return positions.is_cuda and all(torch.is_tensor(t) and t.device == positions.device for t in others)
+
+
 def _supported_call(positions, edge_index, shifts):
-    return (torch.is_tensor(positions) and positions.is_cuda and positions.dtype == torch.float32
-            and positions.dim() == 2 and torch.is_tensor(shifts) and shifts.dtype == torch.float32
-            and torch.is_tensor(edge_index) and edge_index.is_cuda and edge_index.dim() == 2 and edge_index.shape[0] == 2
-            and shifts.shape == (edge_index.shape[1], 3))
+    return (torch.is_tensor(positions) and _together(positions, edge_index, shifts)
+            and positions.dtype == torch.float32 and positions.dim() == 2 and shifts.dtype == torch.float32
+            and edge_index.dim() == 2 and edge_index.shape[0] == 2 and shifts.shape == (edge_index.shape[1], 3))
 
 
 def _wrap(orig):
