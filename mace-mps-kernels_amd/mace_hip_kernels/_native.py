@@ -291,8 +291,12 @@ def ptr(t):
 
 def stream_of(t):
     """The current stream of a GPU tensor's device.  The raw handle: a torch.cuda.Stream object per launch was 3 us of
-    host time, about 100 us of an eager energy and forces call of 34 launches (1.1 ms of host work in all)."""
-    return torch._C._cuda_getCurrentRawStream(t.get_device())
+    host time, about 100 us of an eager energy and forces call of 34 launches (1.1 ms of host work in all).  A host
+    tensor (device index -1, which the raw call takes for the current GPU) is refused as the object's making did."""
+    device = t.get_device()
+    if device < 0:
+        raise ValueError(f'mace_hip_kernels: a kernel was given a tensor on {t.device}; a GPU tensor is expected')
+    return torch._C._cuda_getCurrentRawStream(device)
 
 
 # ------------------------------------------------------------------------------------------- graph capture

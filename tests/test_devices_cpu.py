@@ -6,7 +6,7 @@ import pytest
 import torch
 from torch._subclasses.fake_tensor import FakeTensorMode
 
-from mace_hip_kernels import geometry as G
+from mace_hip_kernels import _native, geometry as G
 
 
 def _inputs():
@@ -39,3 +39,9 @@ def test_strain_needs_its_shapes(change):
     with FakeTensorMode():
         t[name] = torch.empty(shape, dtype=t[name].dtype, device='cuda')
     assert not G._supported_displacement(**t)
+
+
+def test_host_tensors_have_no_stream():
+    """The stream of a launch is asked of one of its operands: a host tensor raises before the kernel gets its pointer."""
+    with pytest.raises(ValueError, match='cpu'):
+        _native.stream_of(torch.empty(1))
