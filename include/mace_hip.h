@@ -417,7 +417,7 @@ int mh_geom_segsum(mh_module* m, const float* g, const int32_t* perm, const int6
  * rowptr [n + 1] and perm, perm[rowptr[seg[b]]] .. perm[rowptr[seg[b + 1]] - 1].  out [B slices, 9]: each of the
  * `slices` workgroups of a segment writes its own row.  For the edges: left = unit, g = dL/dosh, the sender CSR.
  * For the atoms (left = pos, g = dL/dopos, one slice): cell, parts (the edges' [B nparts, 9]) and disp given, out is
- * dL/ddisp [B, 9] and gleft [n, 3] dL/dpos.  Uses MH_GEOM_SEGSUM.
+ * dL/ddisp [B, 9] and gleft [n, 3] dL/dpos (every row's, by its structure batch[row], int64).  Uses MH_GEOM_SEGSUM.
  *
  * mh_geom_det: out[b] = det of the 3x3 matrix a[b] (a [B, 9]), expanded in float64.  Bind MH_GEOM_DET with 256 threads
  * and rows_per_block 256.  No reference counterparts. */
@@ -426,7 +426,8 @@ int mh_geom_strain(mh_module* m, const float* pos, const float* unit, const floa
                    void* stream);
 int mh_geom_strain_sum(mh_module* m, const float* left, const float* g, const int32_t* perm, const int64_t* seg,
                        const int32_t* rowptr, int32_t n, float* out, int32_t slices, const float* cell,
-                       const float* parts, int32_t nparts, const float* disp, float* gleft, int32_t B, void* stream);
+                       const float* parts, int32_t nparts, const float* disp, float* gleft, const int64_t* batch,
+                       int32_t B, void* stream);
 int mh_geom_det(mh_module* m, const float* a, float* out, int32_t B, void* stream);
 /* The sum of rows (mh_geom_segsum) for one column, out[b] = sum of g[seg[b]] .. g[seg[b + 1] - 1] (g [M], seg [B + 1] int64, out [B]):
  * MACE's per-structure energy sums (scatter_sum of the node energies by the sorted batch vector), deterministic

@@ -146,7 +146,7 @@ extern "C" {
 
 const char* mh_last_error(void) { return g_err.c_str(); }
 
-int mh_version(void) { return 45; }
+int mh_version(void) { return 46; }
 
 int mh_launch_log(int enable) {
     std::lock_guard<std::mutex> lock(g_log_mu);
@@ -801,8 +801,10 @@ int mh_geom_segsum(mh_module* m, const float* g, const int32_t* perm, const int6
     const float* none = nullptr;
     const int32_t* rowptr = nullptr;
     float* gleft = nullptr;
+    const int64_t* batch = nullptr;
     int32_t n = 0, slices = 1, nparts = 0;
-    void* args[] = {&g, &perm, &seg, &out, &B, &none, &rowptr, &n, &slices, &none, &none, &nparts, &none, &gleft};
+    void* args[] = {&g, &perm, &seg, &out, &B, &none, &rowptr, &n, &slices, &none, &none, &nparts, &none, &gleft,
+                    &batch};
     return launch(m, MH_GEOM_SEGSUM, B, args, stream, "mh_geom_segsum");
 }
 
@@ -819,14 +821,17 @@ int mh_geom_strain(mh_module* m, const float* pos, const float* unit, const floa
 
 int mh_geom_strain_sum(mh_module* m, const float* left, const float* g, const int32_t* perm, const int64_t* seg,
                        const int32_t* rowptr, int32_t n, float* out, int32_t slices, const float* cell,
-                       const float* parts, int32_t nparts, const float* disp, float* gleft, int32_t B, void* stream) {
+                       const float* parts, int32_t nparts, const float* disp, float* gleft, const int64_t* batch,
+                       int32_t B, void* stream) {
     if (B < 0 || n < 0 || slices < 1 || nparts < 0) return fail(-1, "mh_geom_strain_sum: bad size");
     if (static_cast<int64_t>(B) * slices > 0x7fffffff) return fail(-1, "mh_geom_strain_sum: launch too large");
     if (!left) return n ? fail(-1, "mh_geom_strain_sum: NULL left") : 0;
     if (B > 0 && (!g || !seg || !out)) return fail(-1, "mh_geom_strain_sum: NULL operand");
     if (cell && (slices != 1 || nparts < 1 || !parts)) return fail(-1, "mh_geom_strain_sum: bad epilogue");
-    if (gleft && !disp) return fail(-1, "mh_geom_strain_sum: gleft needs disp");
-    void* args[] = {&g, &perm, &seg, &out, &B, &left, &rowptr, &n, &slices, &cell, &parts, &nparts, &disp, &gleft};
+    if (gleft && (!disp || !batch || perm || rowptr || slices != 1))
+        return fail(-1, "mh_geom_strain_sum: gleft needs disp, batch and plain segments in one slice");
+    void* args[] = {&g, &perm, &seg, &out, &B, &left, &rowptr, &n, &slices, &cell, &parts, &nparts, &disp, &gleft,
+                    &batch};
     return launch(m, MH_GEOM_SEGSUM, static_cast<int64_t>(B) * slices, args, stream, "mh_geom_strain_sum");
 }
 

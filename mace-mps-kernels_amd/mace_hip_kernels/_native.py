@@ -30,7 +30,7 @@ MH_CONV_FWD, MH_CONV_BWD, MH_CONV_BWD_WY, MH_SC_FWD, MH_SC_BWD, MH_CONV_BWD_R, M
     MH_EDGE_BWD, MH_MLP_BWD_P, MH_LIN_BWD_SUM, MH_MLP_H3T, MH_CONV_BWD_T, \
     MH_GEOM_STRAIN, MH_GEOM_DET, MH_MLP_BWD_W = range(84)
 MH_WANT_GX, MH_WANT_GWY, MH_CUT_MASKED, MH_CUT_NOZERO = 1, 2, 4, 8
-ABI_VERSION = 45
+ABI_VERSION = 46
 
 # hipcc/hipRTC options for every generated layer: gfx950 code, -O3, and packed-FP32 instructions disabled.
 ARCH = os.environ.get('MACE_HIP_ARCH', 'gfx950')
@@ -122,7 +122,7 @@ _SIGS = {
     'mh_sc_bwd': (ctypes.c_int, [_P] * 6 + [_I, _P]),
     'mh_geom_segsum': (ctypes.c_int, [_P] * 5 + [_I, _P]),
     'mh_geom_strain': (ctypes.c_int, [_P] * 9 + [_I, ctypes.c_int64, _I, _P]),
-    'mh_geom_strain_sum': (ctypes.c_int, [_P] * 6 + [_I, _P, _I, _P, _P, _I, _P, _P, _I, _P]),
+    'mh_geom_strain_sum': (ctypes.c_int, [_P] * 6 + [_I, _P, _I, _P, _P, _I, _P, _P, _P, _I, _P]),
     'mh_geom_det': (ctypes.c_int, [_P] * 3 + [_I, _P]),
     'mh_mlp_jvp': (ctypes.c_int, [_P] * 6 + [ctypes.c_int64, _P]),
     'mh_mlp_bwd2': (ctypes.c_int, [_P] * 7 + [ctypes.c_int64, _P]),

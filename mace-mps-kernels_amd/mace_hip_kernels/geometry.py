@@ -143,16 +143,31 @@ extern "C" __global__ __launch_bounds__(BLOCK) void geom_jvp(const float* __rest
 // of g[row] (9 wide) or, with ``left``, of the outer product left[row] x g[row] (3 wide each: formed here, a [rows, 9]
 // product written and read back was four launches).  ``slices`` workgroups per segment, each writing its own out row;
 // every thread sums a fixed stride of rows, then a fixed-order tree: deterministic, no atomics.  ``gleft`` gets
-// g + sym g of each row.  With ``cell`` (one slice) the workgroup ends with dL/dsym = sum + cell^T G, G the sum of the
-// ``nparts`` rows of ``parts``, and writes its symmetric part, dL/ddisplacement.
+// g + sym g of each of the n rows by its structure in ``batch``, also of rows in no segment (segments cover every row
+// from the first one's start to the last one's end, so the first and the last workgroup take the rest).  With ``cell``
+// (one slice) the workgroup ends with dL/dsym = sum + cell^T G, G the sum of the ``nparts`` rows of ``parts``, and
+// writes its symmetric part, dL/ddisplacement.
 // Bound by the serial chain of a thread's rows: 1,024 threads per segment, 5.5 rows each on a 160-atom structure.
 #define SEG_K 9
 #define SEG_BLOCK 1024
+// out[row] = g + sym g with the strain of structure s (NaN outside -B .. B - 1, as in geom_strain).
+__device__ __forceinline__ void geom_strained(const float* __restrict__ g, const float* __restrict__ disp, long long s,
+    int B, long long row, float* __restrict__ out) {
+  if (s < 0) s += B;
+  const bool ok = s >= 0 && s < B;
+  const float* d = disp + (ok ? s : 0) * 9;
+  for (int k = 0; k < 3; ++k) {
+    float v = 0.f;
+    for (int a = 0; a < 3; ++a) v += 0.5f * (d[3 * k + a] + d[3 * a + k]) * g[3 * row + a];
+    out[3 * row + k] = ok ? g[3 * row + k] + v : __builtin_nanf("");
+  }
+}
+
 extern "C" __global__ __launch_bounds__(SEG_BLOCK) void geom_segsum(const float* __restrict__ g,
     const int* __restrict__ perm, const long long* __restrict__ seg, float* __restrict__ out, int B,
     const float* __restrict__ left, const int* __restrict__ rowptr, int n, int slices,
     const float* __restrict__ cell, const float* __restrict__ parts, int nparts, const float* __restrict__ disp,
-    float* __restrict__ gleft) {
+    float* __restrict__ gleft, const long long* __restrict__ batch) {
   const int b = blockIdx.x / slices, sl = blockIdx.x - b * slices;
   if (b >= B) return;
   long long lo = seg[b], hi = seg[b + 1];
@@ -178,7 +193,9 @@ extern "C" __global__ __launch_bounds__(SEG_BLOCK) void geom_segsum(const float*
       acc[0] += a0 * g0; acc[1] += a0 * g1; acc[2] += a0 * g2;
       acc[3] += a1 * g0; acc[4] += a1 * g1; acc[5] += a1 * g2;
       acc[6] += a2 * g0; acc[7] += a2 * g1; acc[8] += a2 * g2;
-      if (gleft) {
+      if (gleft && batch[row] != b) {
+        geom_strained(g, disp, batch[row], B, row, gleft);
+      } else if (gleft) {
         gleft[3 * row] = g0 + (sym[0] * g0 + sym[1] * g1 + sym[2] * g2);
         gleft[3 * row + 1] = g1 + (sym[3] * g0 + sym[4] * g1 + sym[5] * g2);
         gleft[3 * row + 2] = g2 + (sym[6] * g0 + sym[7] * g1 + sym[8] * g2);
@@ -186,6 +203,12 @@ extern "C" __global__ __launch_bounds__(SEG_BLOCK) void geom_segsum(const float*
     } else {
       for (int k = 0; k < SEG_K; ++k) acc[k] += g[row * SEG_K + k];
     }
+  }
+  if (gleft) {                     // the rows before the first segment and after the last (none as a rule)
+    if (b == 0)
+      for (long long row = threadIdx.x; row < lo; row += SEG_BLOCK) geom_strained(g, disp, batch[row], B, row, gleft);
+    if (b == B - 1)
+      for (long long row = hi + threadIdx.x; row < n; row += SEG_BLOCK) geom_strained(g, disp, batch[row], B, row, gleft);
   }
   __shared__ float red[SEG_BLOCK / 64][SEG_K], tot[SEG_K];
   for (int k = 0; k < SEG_K; ++k) {
@@ -515,7 +538,7 @@ class _StrainFn(torch.autograd.Function):
         P = _native.ptr
         _native.launch('geom_strain', _native.load().mh_geom_strain, _module(p.device).handle, P(p), P(u), P(c), P(D),
                        P(batch), P(gr.send), P(opos), P(osh), N, E, B, _native.stream_of(p))
-        ctx.save_for_backward(D, p, u, c, ptr)
+        ctx.save_for_backward(D, p, u, c, batch, ptr)
         ctx.gr = gr
         return opos, osh
 
@@ -523,7 +546,7 @@ class _StrainFn(torch.autograd.Function):
     def backward(ctx, gp, gs):
         if torch.is_grad_enabled():          # only true under create_graph=True
             raise RuntimeError(_DOUBLE_BACKWARD)
-        D, p, u, c, ptr = ctx.saved_tensors
+        D, p, u, c, batch, ptr = ctx.saved_tensors
         N, E, B = p.shape[0], u.shape[0], D.shape[0]
         gp, gs = gp.contiguous(), gs.contiguous()
         rp_s, ei_s = ctx.gr.by_send()
@@ -538,9 +561,9 @@ class _StrainFn(torch.autograd.Function):
         # dL/dcell' = sum of unit_shift x g_shift over the structure's edges, then dL/dsym over its atoms
         if E:
             _native.launch('geom_segsum', lib.mh_geom_strain_sum, m, P(u), P(gs), P(ei_s), P(ptr), P(rp_s), N,
-                           P(parts), slices, None, None, 0, None, None, B, st)
+                           P(parts), slices, None, None, 0, None, None, None, B, st)
         _native.launch('geom_segsum', lib.mh_geom_strain_sum, m, P(p), P(gp), None, P(ptr), None, N, P(gD), 1, P(c),
-                       P(parts), slices, P(D), P(gpos), B, st)
+                       P(parts), slices, P(D), P(gpos), P(batch), B, st)
         return gD, gpos, None, None, None, None, None
 
 

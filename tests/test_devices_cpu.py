@@ -19,6 +19,8 @@ def _inputs():
 @pytest.mark.parametrize('name', ['positions', 'unit_shifts', 'cell', 'edge_index', 'batch', 'ptr'])
 @pytest.mark.parametrize('device', ['cpu', 'cuda:1'])
 def test_strain_and_geometry_need_one_device(name, device):
+    if device == 'cuda:1' and torch.cuda.device_count() == 1:
+        pytest.skip('a stand-in of a second GPU: none on this machine, and one is not made beside a first')
     t = _inputs()
     assert G._supported_displacement(**t)
     assert G._supported_call(t['positions'], t['edge_index'], t['unit_shifts'])

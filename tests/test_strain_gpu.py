@@ -95,3 +95,27 @@ def test_a_gradient_in_cell_or_unit_shifts_keeps_the_expressions(needs):
     for a, b in zip(torch.autograd.grad((s * w).sum() + (p ** 2).sum(), [t[needs], d, pos]),
                     torch.autograd.grad((s2 * w).sum() + (p2 ** 2).sum(), [t[needs], d2, pos])):
         assert torch.allclose(a, b, atol=2e-4), (a - b).abs().max()
+
+
+@pytest.mark.parametrize('ptr', [[0, 4, 7], [2, 4, 9], [3, 3, 5], [0, 0, 0], [8, 5, 2]])
+def test_atoms_outside_ptr_keep_their_gradient(ptr):
+    """A ptr that does not cover every atom: dL/dpositions is MACE's expression at every atom, whichever segments the
+    displacement's own gradient sums."""
+    print(f'[case] strain, atoms outside ptr {ptr}', flush=True)
+    dev = torch.device('cuda:0')
+    g = torch.Generator().manual_seed(7)
+    n, B = 9, 2
+    batch = torch.tensor([0] * 4 + [1] * 5)
+    pos, D = torch.randn(n, 3, generator=g), torch.randn(B, 3, 3, generator=g) * 0.02
+    ei = torch.randint(0, n, (2, 30), generator=g)
+    gp = torch.randn(n, 3, generator=g)
+    d, p = D.double().requires_grad_(True), pos.double().requires_grad_(True)
+    sym = 0.5 * (d + d.transpose(-1, -2))
+    want, = torch.autograd.grad(p + torch.einsum('be,bec->bc', p, sym[batch]), p, gp.double())
+    torch.full((64, 3), float('nan'), device=dev)              # (freed: what unwritten rows would hold)
+    d, p = D.to(dev).requires_grad_(True), pos.to(dev).requires_grad_(True)
+    op, _ = G._StrainFn.apply(d, p, torch.zeros(30, 3, device=dev), torch.eye(3, device=dev).repeat(B, 1, 1),
+                              batch.to(dev), torch.tensor(ptr, device=dev), C.graph_for(ei.to(dev), n))
+    got, = torch.autograd.grad(op, p, gp.to(dev))
+    # a sum of four products of values below 5
+    assert (got.double().cpu() - want).abs().max() <= 4 * 5 * 1.2e-7, (got.cpu(), want)
