@@ -627,7 +627,8 @@ def _bwd_recv(G, gyr, pdecl, decl, copy, cut=False, tan=False):
     ]
     L += G.ld_g('  ', 'r', 'gv')
     L += ['  ' + decl('xn', nx), '  ' + decl('wn', nk)] + (['  ' + decl('tn', nk)] if tan else [])
-    if BWD_PREFETCH > 1:
+    pf = 1 if tan else BWD_PREFETCH      # (tan: one stage, its rows of T are as many registers again)
+    if pf > 1:
         L += ['  ' + decl('xm', nx), '  ' + decl('wm', nk)]
     nt = W_NT_BWD and not tan            # (tan: each shared row of W0 and of T is read twice)
 
@@ -679,7 +680,7 @@ def _bwd_recv(G, gyr, pdecl, decl, copy, cut=False, tan=False):
         C += ['    {', '      const int er0 = mh_bcast(my_w, 0), s0 = mh_bcast(my_s, 0);']
         C += G.ld_x('      ', 's0', 'xn') + ld_rows('      ', 'er0')
         C += ['    }']
-        if BWD_PREFETCH > 1:          # edge 1 (or the last edge again) one stage further out
+        if pf > 1:          # edge 1 (or the last edge again) one stage further out
             C += ['    {', '      const int er1 = mh_bcast(my_w, min(1, cnt - 1)), s1 = mh_bcast(my_s, min(1, cnt - 1));']
             C += G.ld_x('      ', 's1', 'xm') + G.ld_w('      ', 'er1', 'wm', W_NT_BWD)
             C += ['    }']
@@ -695,7 +696,7 @@ def _bwd_recv(G, gyr, pdecl, decl, copy, cut=False, tan=False):
             C += ['      float Pc = 0.0f;']
         else:
             C += copy('w', 'wn', nk)
-        if BWD_PREFETCH > 1:
+        if pf > 1:
             C += [f'      xn{i} = xm{i};' for i in range(nx)] + [f'      wn{k} = wm{k};' for k in range(nk)]
             C += ['      {', '        const int j2 = min(j + 2, cnt - 1);',
                   '        const int er2 = mh_bcast(my_w, j2), s2 = mh_bcast(my_s, j2);']
