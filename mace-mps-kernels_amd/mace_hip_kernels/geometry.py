@@ -354,10 +354,14 @@ class _GeomFn(torch.autograd.Function):
         vec = torch.empty(E, 3, device=p.device, dtype=torch.float32)
         ln = torch.empty(E, 1, device=p.device, dtype=torch.float32)
         if edge_ops is not None:
-            # the harmonics and the embedding of the same edges in the same pass, left on vec for those modules
+            # the harmonics and the embedding of the same edges in the same pass, left on vec for those modules; the
+            # derivatives in the length only where a convolution may take them (conv_mlp.length_tangents: not with a
+            # gradient of the shifts, as stress has, and not for a double backward)
             from . import edgefeat
-            edgefeat.forward_all(p, gr, sh, vec, ln, edge_ops, tangents=ctx.needs_input_grad[0] and _conv.PAIR_GRADS
-                                 and _conv.LENGTH_GRADS and E >= _conv.EDGE_COMPACT_MIN)
+            edgefeat.forward_all(p, gr, sh, vec, ln, edge_ops,
+                                 tangents=ctx.needs_input_grad[0] and not ctx.needs_input_grad[1]
+                                 and not double_backward and _conv.PAIR_GRADS and _conv.LENGTH_GRADS
+                                 and E >= _conv.EDGE_COMPACT_MIN)
         else:
             mod = _module(p.device)
             _native.launch('geom_fwd', _native.load().mh_geom_fwd, mod.handle, _native.ptr(p), _native.ptr(gr.send),
