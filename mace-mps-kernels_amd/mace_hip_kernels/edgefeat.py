@@ -191,6 +191,9 @@ class _EdgeFeatFn(torch.autograd.Function):
         sh_op, emb_op, _, Y, feats, cut = made[:6]
         ctx.save_for_backward(vec, ln)
         ctx.sh_op, ctx.emb_op, ctx.nslot = sh_op, emb_op, nslot
+        # an output without a gradient arrives as None: autograd would fill zeros for each (a launch, and edge_bwd reads
+        # them), and a convolution that gives its gradient to a lengths alias gives none to the features and the cutoff
+        ctx.set_materialize_grads(False)
         extra = []
         for _ in range(nslot):
             extra += [Y.detach(), feats.detach(), cut.detach()]

@@ -1,6 +1,6 @@
 """
 The autograd side of the gradients to the edge lengths, on the CPU with the launches recorded instead of run: when the
-edge pass forms the features' derivatives in the length.
+edge pass forms the features' derivatives in the length, and which gradients its backward is given.
 """
 import pytest
 import torch
@@ -22,3 +22,30 @@ def test_derivatives_are_formed_where_a_convolution_takes_them(monkeypatch, grad
     shifts = torch.zeros(edges, 3, requires_grad=grad_shifts)
     G._GeomFn.apply(pos, shifts, torch.zeros(2, edges, dtype=torch.int64), double_backward, ('harmonics', 'embedding'))
     assert asked == [want]
+
+
+class _Op:
+    double_backward = False
+
+
+def _joint(nslot, nlen, E=5):
+    vec, ln = torch.ones(E, 3, requires_grad=True), torch.ones(E, 1, requires_grad=True)
+    made = (_Op, _Op, ln, torch.ones(E, 4), torch.ones(E, 8), torch.ones(E, 1))
+    return vec, ln, edgefeat._EdgeFeatFn.apply(vec, ln, made, nslot, nlen)
+
+
+@pytest.mark.parametrize('used', [('Y', 'len0', 'Y1', 'len1'), ('Y', 'f', 'c'), ('f1', 'len0'), ('len1',)])
+def test_outputs_without_a_gradient_reach_the_backward_as_none(monkeypatch, used):
+    """Only what a consumer gave is handed on: no zeros are formed in the place of the others."""
+    seen = []
+
+    def bwd(sh_op, emb_op, vec, ln, *lists):
+        seen.extend(lists)
+        return torch.zeros_like(vec), torch.zeros_like(ln)
+    monkeypatch.setattr(edgefeat, '_edge_bwd', bwd)
+    vec, ln, outs = _joint(1, 2)
+    names = ['Y', 'f', 'c', 'Y1', 'f1', 'c1', 'len0', 'len1']
+    outs = dict(zip(names, outs))
+    torch.autograd.grad(sum(outs[k].sum() for k in used), [vec, ln])
+    for gs, keys in zip(seen, (('Y', 'Y1'), ('f', 'f1'), ('c', 'c1'), ('len0', 'len1'))):
+        assert [g is not None for g in gs] == [k in used for k in keys]
