@@ -818,7 +818,8 @@ PAIR_RADIAL = True
 PAIR_GRADS = True
 # ... and, when the patched edge pass also made the features' derivatives in the length, dL/dW0 is not formed at all:
 # the MLP's backward forms the rows' derivatives in the length, and the convolution's reduces each edge's dL/dlength
-# against them (mh_mlp_tangents, mh_conv_bwd_len)
+# against them (mh_mlp_tangents, mh_conv_bwd_len).  Off for a model whose own forward asks for the gradient of its edge
+# features beside the positions': while it runs, only hooks and retain_grad on them are seen (edgefeat.Watch)
 LENGTH_GRADS = True
 
 

@@ -670,14 +670,14 @@ class ConvRadialFn(torch.autograd.Function):
     and so the forces, are those of the per-edge backward to fp32 rounding, while the split between the two edges
     is not kept (the partner's row is zero).
 
-    With a lengths alias ``ln`` and ``tan`` = (dfeats/dr, dcutoff/dr, the lengths' grad_fn) (``length_tangents``) the
-    gradient goes to the lengths instead of to ef and cut: the weights are a function W0(r) c(r) of each edge's length,
-    so dL/dr[e] = sum_k,u dL/d(W0 c)[e, k, u] (c dW0/dr + c' W0), which the convolution's backward reduces in registers
+    With a lengths alias ``ln`` and ``tan`` = (dfeats/dr, dcutoff/dr, the lengths' grad_fn, a Watch)
+    (``length_tangents``) the gradient goes to the lengths instead of to ef and cut: the weights are a function
+    W0(r) c(r) of each edge's length, so dL/dr[e] = sum_k,u dL/d(W0 c)[e, k, u] (c dW0/dr + c' W0), which the convolution's backward reduces in registers
     (``conv_bwdt``) against rows of dW0/dr, formed from the hidden layers' derivatives in r by the forward's output
     kernel, one row per edge and its reverse.  dL/dW0 is neither stored nor projected (1280 weights, 78k edges of 39k
-    rows: the projection's 140 us become 27 + 55).  A backward that wants the gradients of ef or cut themselves (the
-    lengths' own producer not run by it) takes the form above.  No double backward: the two-kernel modules take that
-    (``patch_model(double_backward=True)``)."""
+    rows: the projection's 140 us become 27 + 55).  A backward that may want the gradients of ef or cut themselves (the
+    lengths' own producer not run by it, or ``edgefeat.Watch.wanted``) takes the form above.  No double
+    backward: the two-kernel modules take that (``patch_model(double_backward=True)``)."""
 
     @staticmethod
     def forward(ctx, x, Y, ef, cut, edge_index, op, ln=None, tan=None):
@@ -700,7 +700,8 @@ class ConvRadialFn(torch.autograd.Function):
             raise ValueError('graph too large for int32 indices')
         masked = C._support_masked(cut) and op.skip_masked
         xc, Yc = x.contiguous(), Y.contiguous()
-        efc, cutf = ef.reshape(E, -1).contiguous(), cut.reshape(-1).contiguous()
+        # (detached: a view would hold ef and cut themselves, which edgefeat.Watch counts the holders of)
+        efc, cutf = ef.detach().reshape(E, -1).contiguous(), cut.detach().reshape(-1).contiguous()
         rows = count = wrow = partner = frows = fcount = None
         gr = C.graph_for(edge_index, n)
         if masked and E >= C.EDGE_COMPACT_MIN:
@@ -740,7 +741,7 @@ class ConvRadialFn(torch.autograd.Function):
         none = (None,) * 4
         if not (want_x or want_y or want_ef or want_cut):
             return (None,) * 4 + none
-        if ctx.tan is not None and _executes(ctx.tan[2]):
+        if ctx.tan is not None and _executes(ctx.tan[2]) and not ctx.tan[3].wanted():
             gx, gY, glen = ConvRadialFn._to_lengths(ctx, g.contiguous(), want_x)
             return gx, gY if want_y else None, None, None, None, None, glen.view(ctx.ln_shape), None
         compact = ctx.rows is not None
@@ -767,7 +768,7 @@ class ConvRadialFn(torch.autograd.Function):
         op, gr, s = ctx.op, ctx.gr, ctx.op.spec
         mlp = op.deferred_mlp()
         rows, count, _ = ctx.pairs
-        dfeats, dcut, _ = ctx.tan
+        dfeats, dcut = ctx.tan[:2]
         E, n = Y.shape[0], x.shape[0]
         T = mlp_rows(mlp, mlp_tangents(mlp, ef, dfeats, rows, count), rows, count)
         gx = torch.empty_like(x) if want_x else None
@@ -784,8 +785,8 @@ class ConvRadialFn(torch.autograd.Function):
 
 
 def length_tangents(w, mlp):
-    """(lengths alias, (dfeats, dcutoff, the lengths' grad_fn)) for ``ConvRadialFn`` on the unformed weights ``w`` (a
-    ``FusedWeights`` of ``mlp``), or nothing where its gradient to the lengths does not apply: fewer edges than the row
+    """(lengths alias, (dfeats, dcutoff, the lengths' grad_fn, Watch)) for ``ConvRadialFn`` on the unformed weights ``w``
+    (a ``FusedWeights`` of ``mlp``), or nothing where its gradient to the lengths does not apply: fewer edges than the row
     lists pay for, the pairing switched off, gradients off, lengths whose split between an edge and its reverse matters
     (``geometry.lengths_pair_symmetric``), an MLP the weight-stationary output kernel does not cover, or no derivatives
     left by the edge pass (``edgefeat.length_slot``)."""

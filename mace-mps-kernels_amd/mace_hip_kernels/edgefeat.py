@@ -14,6 +14,7 @@ gradient and dL/dlengths from the embedding's, in one pass (the statements of ``
 Outputs left on a tensor are taken only by the module they were made for, only once, and only while the tensor is
 unmodified (same version); any other call computes as before.
 """
+import sys
 import weakref
 
 import torch
@@ -240,25 +241,54 @@ def take_harmonics(sh_op, vec):
         for k, t in enumerate((Y, feats, cut)):
             set_slots(t, outs[3 + k:3 + 3 * nslot:3])
     if nlen:
-        # (the lengths' own producer tells a backward whether dL/dlength is wanted at all)
-        feats._mh_len = (feats._version, weakref.ref(cut), cut._version, made[8], made[9], list(outs[-nlen:]), ln.grad_fn)
+        # (the lengths' own producer tells a backward whether dL/dlength is wanted at all; one Watch, made on demand and
+        # held by the convolutions' nodes alone, serves them all)
+        feats._mh_len = (feats._version, weakref.ref(cut), cut._version, made[8], made[9], list(outs[-nlen:]), ln.grad_fn,
+                         [None])
     ln._mh_emb = (made[1], feats, cut, ln._version)
     return Y
 
 
+def _hooked(t):
+    return bool(t._backward_hooks) or t.retains_grad
+
+
+class Watch:
+    """The features and the cutoff whose gradients a convolution leaves out when it gives the lengths', held so that its
+    backward can tell whether someone came to want them after its forward: by a hook or retain_grad on either, or, once
+    the model's call has returned (its own locals gone), by still holding one, as ``autograd.grad(E, [positions,
+    edge_feats])`` needs (the engine does not tell a node which outputs a pass captures)."""
+
+    def __init__(self, feats, cut, call):
+        self.feats, self.cut, self.call = feats, cut, call
+
+    def wanted(self):
+        if _hooked(self.feats) or _hooked(self.cut):
+            return True
+        if self.call is not None and self.call.running:
+            return False
+        # this object's reference and getrefcount's argument
+        return sys.getrefcount(self.feats) > 2 or sys.getrefcount(self.cut) > 2
+
+
 def length_slot(feats, cut):
-    """(lengths alias, dfeats/dlength, dcutoff/dlength, the lengths' grad_fn) for a consumer of the joint node's features
-    and cutoff that forms dL/dlength itself (its gradient goes to the alias, none to the features and the cutoff): where
-    the node left one, both tensors are unmodified, and nothing watches their own gradients (a hook, retain_grad);
-    else None."""
+    """(lengths alias, dfeats/dlength, dcutoff/dlength, the lengths' grad_fn, Watch) for a consumer of the joint node's
+    features and cutoff that forms dL/dlength itself (its gradient goes to the alias, none to the features and the
+    cutoff): where the node left one, both tensors are unmodified, and nothing watches their own gradients (a hook,
+    retain_grad); else None.  Its backward asks the Watch again."""
+    from .geometry import running_call
     feats, cut = stash_owner(feats), stash_owner(cut)
     m = getattr(feats, '_mh_len', None)
     if (m is None or m[0] != feats._version or m[1]() is not cut or m[2] != cut._version or not m[5]
             or not m[5][0].requires_grad or m[6] is None):
         return None
-    if any(t._backward_hooks or t.retains_grad for t in (feats, cut)):
+    if _hooked(feats) or _hooked(cut):
         return None
-    return m[5].pop(0), m[3], m[4], m[6]
+    watch = m[7][0]() if m[7][0] is not None else None
+    if watch is None:
+        watch = Watch(feats, cut, running_call())
+        m[7][0] = weakref.ref(watch)             # (weak: the Watch holds feats)
+    return m[5].pop(0), m[3], m[4], m[6], watch
 
 
 def take_embedding(emb_op, ln):

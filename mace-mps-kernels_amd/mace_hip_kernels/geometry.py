@@ -49,6 +49,7 @@ _PTR = contextvars.ContextVar('mace_hip_kernels_geometry_ptr', default=None)   #
 _BATCH = contextvars.ContextVar('mace_hip_kernels_geometry_batch', default=None)  # the batch vector, likewise
 # (harmonics, embedding) drop-ins of the running forward whose outputs the geometry's forward makes too (edgefeat)
 _EDGE = contextvars.ContextVar('mace_hip_kernels_geometry_edge', default=None)
+_CALL = contextvars.ContextVar('mace_hip_kernels_geometry_call', default=None)    # the Call of a running forward
 FUNCTION = 'get_edge_vectors_and_lengths'
 DISPLACEMENT = 'get_symmetric_displacement'
 SCATTER = 'scatter_sum'
@@ -733,7 +734,18 @@ def _edge_ops(model):
     return None
 
 
+class Call:
+    """One forward of a patched model: ``running`` until it returns (read by its backward, in autograd's threads)."""
+    running = True
+
+
+def running_call():
+    return _CALL.get()
+
+
 def _forward_with_geometry(self, *args, **kwargs):
+    call = Call()
+    token_call = _CALL.set(call)
     token = _ACTIVE.set('double_backward' if getattr(self, '_mh_geometry_double_backward', False) else True)
     token_edge = _EDGE.set(_edge_ops(self))
     data = args[0] if args else kwargs.get('data')
@@ -743,10 +755,12 @@ def _forward_with_geometry(self, *args, **kwargs):
     try:
         return type(self).forward(self, *args, **kwargs)
     finally:
+        call.running = False
         _BATCH.reset(token_batch)
         _PTR.reset(token_ptr)
         _EDGE.reset(token_edge)
         _ACTIVE.reset(token)
+        _CALL.reset(token_call)
 
 
 def install(model):

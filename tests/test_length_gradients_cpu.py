@@ -1,6 +1,7 @@
 """
 The autograd side of the gradients to the edge lengths, on the CPU with the launches recorded instead of run: when the
-edge pass forms the features' derivatives in the length, and which gradients its backward is given.
+edge pass forms the features' derivatives in the length, which gradients its backward is given, and what a convolution's
+backward can tell of a wish for the gradients it leaves out.
 """
 import pytest
 import torch
@@ -49,3 +50,40 @@ def test_outputs_without_a_gradient_reach_the_backward_as_none(monkeypatch, used
     torch.autograd.grad(sum(outs[k].sum() for k in used), [vec, ln])
     for gs, keys in zip(seen, (('Y', 'Y1'), ('f', 'f1'), ('c', 'c1'), ('len0', 'len1'))):
         assert [g is not None for g in gs] == [k in used for k in keys]
+
+
+def _watched():
+    call = G.Call()
+    vec, ln, (Y, f, c, *_) = _joint(0, 0)
+    return call, edgefeat.Watch(f, c, call), f, c
+
+
+def test_nobody_holds_the_features():
+    call, watch, f, c = _watched()
+    assert not watch.wanted()                       # held by the running forward's locals
+    call.running = False
+    assert watch.wanted()
+    del f
+    assert watch.wanted()
+    del c
+    assert not watch.wanted()
+
+
+@pytest.mark.parametrize('which', [0, 1])
+@pytest.mark.parametrize('how', ['hook', 'retain'])
+def test_late_hooks_are_seen_without_a_holder(which, how):
+    call, watch, *pair = _watched()
+    pair[which].register_hook(lambda g: None) if how == 'hook' else pair[which].retain_grad()
+    assert watch.wanted()
+    call.running = False
+    del pair
+    assert watch.wanted()
+
+
+def test_a_convolutions_own_views_are_not_holders():
+    """As ConvRadialFn keeps them: contiguous rows of the detached tensors."""
+    call, watch, f, c = _watched()
+    kept = f.detach().reshape(5, -1).contiguous(), c.detach().reshape(-1).contiguous()
+    call.running = False
+    del f, c
+    assert not watch.wanted() and len(kept) == 2

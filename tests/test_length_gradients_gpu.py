@@ -180,6 +180,74 @@ def test_gradient_of_the_features_alone(models, monkeypatch):
             assert torch.equal(a, b)
 
 
+def _late(models, monkeypatch, after, wants):
+    """(gradients, whether the backward went to the lengths) of a call whose backward runs after it returned, on and off
+    ``LENGTH_GRADS``: ``after(edge features, cutoff)`` runs between the two, ``wants(batch, kept)`` are the inputs."""
+    _, met = models
+    dev = torch.device('cuda:0')
+    kept, got = [], []
+    h = met.radial_embedding.register_forward_hook(lambda mod, args, out: kept.extend(out))
+    try:
+        for on in (True, False):
+            monkeypatch.setattr(hconv, 'LENGTH_GRADS', on)
+            kept.clear()
+            b = _batch(4, dev)
+            energy = met(b, compute_force=False, training=True)['energy'].sum()
+            also = after(kept)
+            ins = wants(b, kept)
+            grads, sym = _tags(lambda: torch.autograd.grad(energy, ins, allow_unused=True))
+            got.append((list(grads) + list(also()), any(k.startswith('conv_bwdt_') for v in sym.values() for k in v)))
+    finally:
+        h.remove()
+    return got
+
+
+def _equal(a, b):
+    assert len(a) == len(b)
+    for x, y in zip(a, b):
+        assert (x is None) == (y is None) and (x is None or torch.equal(x, y))
+
+
+def test_late_hook_and_retained_gradient(models, monkeypatch):
+    """A hook or retain_grad that comes after the forward, its tensor then dropped: the gradient of the dL/dW0 path."""
+    print('[case] hooks after the forward', flush=True)
+    for how in ('hook', 'retain'):
+        def after(kept):
+            seen = []
+            if how == 'hook':
+                for t in kept:
+                    t.register_hook(lambda g: seen.append(g.detach().clone()))
+                kept.clear()
+                return lambda: seen
+            f, c = kept
+            f.retain_grad(), c.retain_grad()
+            return lambda: [f.grad, c.grad]
+        (a, on), (b, off) = _late(models, monkeypatch, after, lambda batch, kept: [batch['positions']])
+        assert not on and not off and len(a) == 3 and all(t is not None for t in a)
+        _equal(a, b)
+
+
+def test_positions_and_features_together(models, monkeypatch):
+    """autograd.grad towards the positions and the edge features and cutoff in one pass, after the call returned."""
+    print('[case] gradients of the positions and the features', flush=True)
+    (a, on), (b, off) = _late(models, monkeypatch, lambda kept: lambda: [],
+                              lambda batch, kept: [batch['positions'], *kept])
+    assert not on and not off and all(t is not None for t in a)
+    _equal(a, b)
+
+
+def test_backward_after_the_call_still_goes_to_the_lengths(models, monkeypatch):
+    """Nobody holds the features once the call has returned: the fast form, forces as the other's."""
+    print('[case] backward after the call', flush=True)
+
+    def after(kept):
+        kept.clear()
+        return lambda: []
+    (a, on), (b, off) = _late(models, monkeypatch, after, lambda batch, kept: [batch['positions']])
+    assert on and not off
+    _close(a[0], b[0], 2e-6)
+
+
 def test_captured_replays(models):
     """A captured call replayed with eager calls between: every replay as the eager result on the same positions."""
     from mace_hip_kernels.graphs import capture
