@@ -205,7 +205,7 @@ def _kernel_table(met, batch, n_real_edges, summary, symbols):
             rows[f'mlp_fwd[{m.tag}]'] = (bf, s.flops(ef_rows))
             rows[f'mlp_bwd[{m.tag}]'] = (bb, s.flops(ef_rows if getattr(m, 'bwd_paired', False) else eb_rows))
     # (the radial MLP's share of the backward to the lengths: the hidden layers on dual numbers)
-    rows.update({f'mlp_bwd[{tag}]': r for tag, r in lengths.items()})
+    rows.update({f'mlp_tangents[{tag}]': r for tag, r in lengths.items()})
     # edge geometry: positions, shifts and the edge list in, vectors and lengths out; backward: vectors, lengths and
     # their gradients plus both CSRs in, the position gradient out
     E = batch['edge_index'].shape[1]

@@ -790,7 +790,7 @@ def _source(spec, second):
         return H
 
     def h3t_kernel(name):
-        """mlp_bwdp_h: the derivative of ``mlp_h3``'s result in the edge length (the hidden layers on dual numbers, the
+        """mlp_h3t: the derivative of ``mlp_h3``'s result in the edge length (the hidden layers on dual numbers, the
         features ef carrying their derivatives dfe): slot i < count (edge rows[i]) stores dh/dr to ``t3`` at row i, or
         with ``byrow`` at row rows[i].  The output layer over it gives the derivatives of the W0 rows."""
         H = head(name, 'const float* __restrict__ ef, const float* __restrict__ dfe, const float* __restrict__ Wh, '
@@ -969,7 +969,7 @@ def _source(spec, second):
         L += bwd_kernel(spec.kname('mlp_bwdp'), False, paired=True) + walk_kernel(spec.kname('mlp_bwd_w'))
         hidden_only()
         L += h3_kernel(spec.kname('mlp_h3')) + out_kernel(spec.kname('mlp_out'))
-        L += h3t_kernel(spec.kname('mlp_bwdp_h'))
+        L += h3t_kernel(spec.kname('mlp_h3t'))
     return '\n'.join(L)
 
 
@@ -1080,12 +1080,11 @@ def mlp_forward(op, ef, rows=None, count=None):
 
 def mlp_tangents(op, ef, dfeats, rows, count, byrow=False):
     """dh/dr [E, 64]: the derivative of the listed rows' last hidden activations in the edge length, from the features
-    and their derivatives in it (``mlp_bwdp_h``); at slot i for edge rows[i], or with ``byrow`` at row rows[i]."""
+    and their derivatives in it (``mlp_h3t``); at slot i for edge rows[i], or with ``byrow`` at row rows[i]."""
     E = ef.shape[0]
     t3 = torch.empty(E, op.spec.hs[-2], device=ef.device, dtype=torch.float32)
     P = _native.ptr
-    op.bwd_paired = True
-    _native.launch(f'mlp_bwd[{op.tag}]', _native.load().mh_mlp_tangents, op.module.handle, P(ef), P(dfeats), P(op.WhT),
+    _native.launch(f'mlp_tangents[{op.tag}]', _native.load().mh_mlp_tangents, op.module.handle, P(ef), P(dfeats), P(op.WhT),
                    P(t3), E, P(rows), P(count), int(byrow), _native.stream_of(ef))
     return t3
 
@@ -1183,7 +1182,7 @@ class HipRadialMLP(torch.nn.Module):
                 _native.MH_MLP_HIDB: (self.spec.kname('mlp_hidb'), BLOCK, 64 * NB_BWD),
                 _native.MH_MLP_H3: (self.spec.kname('mlp_h3'), BLOCK, 64),
                 _native.MH_MLP_OUT: (self.spec.kname('mlp_out'), BLOCK, 1),
-                _native.MH_MLP_H3T: (self.spec.kname('mlp_bwdp_h'), BLOCK, 64),
+                _native.MH_MLP_H3T: (self.spec.kname('mlp_h3t'), BLOCK, 64),
                 _native.MH_MLP_BWD_W: (self.spec.kname('mlp_bwd_w'), BLOCK, 64),
             })
         self.ncb = -(-self.spec.hs[-1] // WS_COLS)

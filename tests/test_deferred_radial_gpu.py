@@ -413,10 +413,11 @@ def test_patched_model_pairs_bitwise(monkeypatch):
 
 
 def test_patched_model_paired_gradients(monkeypatch):
-    """config 2: the MLP backward over the pairs of exact reverses (conv.PAIR_GRADS, the default) against the
-    per-edge backward: energies bitwise equal, forces to fp32 rounding, and the paired kernel runs for both layers
-    with E+F but not with stress (the shifts then need a gradient of their own)."""
+    """config 2 with the gradients kept off the lengths (conv.LENGTH_GRADS): the MLP backward over the pairs of exact
+    reverses (conv.PAIR_GRADS) against the per-edge backward: energies bitwise equal, forces to fp32 rounding, and the
+    paired kernel runs for both layers with E+F but not with stress (the shifts then need a gradient of their own)."""
     dev = _dev()
+    monkeypatch.setattr(hconv, 'LENGTH_GRADS', False)
     print('[case] patched model, paired radial gradients (config 2)', flush=True)
     model, batch, _ = factory.workload(2)
     b = {k: (v.to(dev) if torch.is_tensor(v) else v) for k, v in batch.items()}

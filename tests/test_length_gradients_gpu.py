@@ -135,6 +135,7 @@ def test_model_forces_and_routes(models, monkeypatch):
     want = ref(_batch(4, dev, torch.float64), compute_force=True)
     new, sym = _tags(lambda: met(_batch(4, dev), compute_force=True))
     assert any(k.startswith('conv_bwdt_') for v in sym.values() for k in v), sym
+    assert not any(k.startswith('mlp_bwd') for v in sym.values() for k in v), sym
     monkeypatch.setattr(hconv, 'LENGTH_GRADS', False)
     old, sym = _tags(lambda: met(_batch(4, dev), compute_force=True))
     assert not any(k.startswith('conv_bwdt_') for v in sym.values() for k in v), sym
@@ -276,7 +277,7 @@ def test_second_layer_energy_only(models):
     print('[case] energy only', flush=True)
     with torch.no_grad():
         a, sym = _tags(lambda: met(_batch(4, dev), compute_force=False))
-    assert not any('mlp_bwd' in k for v in sym.values() for k in v), sym
+    assert not any(k.startswith(('mlp_bwd', 'mlp_h3t')) for v in sym.values() for k in v), sym
     b = met(_batch(4, dev), compute_force=True)
     _close(a['energy'], b['energy'].detach(), 2e-6)
     assert np.isfinite(float(a['energy'].sum()))
