@@ -646,11 +646,11 @@ int mh_edge_bwd_len(mh_module* m, const float* vec, const float* len, const floa
                     const float* glen1, const float* glen2, float* gvec, float* glen, int64_t E, void* stream);
 /* The radial MLP's derivative in the edge length r, for features that are a function of r alone (dfeats [E, n]: their
  * derivatives): slot i < count[0] (edge rows[i]; both NULL: every edge) writes d(last hidden activations)/dr to t3
- * [E, 64] at row i (byrow: at row rows[i]).  mh_mlp_out runs the output layer over such rows in slot order (MH_MLP_OUT, as
- * mh_mlp_fwd_ws does over its h3): rows of dW0/dr.  The gradient of an edge's length is then the dot product of its
+ * [E, 64] at row i.  mh_mlp_out runs the output layer over such rows in slot order (MH_MLP_OUT, as mh_mlp_fwd_ws
+ * does over its h3): rows of dW0/dr.  The gradient of an edge's length is then the dot product of its
  * dL/d(W0 c) row with c dW0/dr + c' W0, and that row is never stored (mh_conv_bwd_len).  No reference counterpart. */
 int mh_mlp_tangents(mh_module* m, const float* ef, const float* dfeats, const float* WhT, float* t3, int64_t E,
-                    const int32_t* rows, const int32_t* count, int32_t byrow, void* stream);
+                    const int32_t* rows, const int32_t* count, void* stream);
 int mh_mlp_out(mh_module* m, const float* h, const uint16_t* Wo, float* W, int64_t E, const int32_t* rows,
                const int32_t* count, int32_t ncb, void* stream);
 /* The receiver-ordered backward with masked edges (mh_conv_bwd_recv_rows, MH_CUT_MASKED) taken to the edge lengths: W and

@@ -146,7 +146,7 @@ extern "C" {
 
 const char* mh_last_error(void) { return g_err.c_str(); }
 
-int mh_version(void) { return 46; }
+int mh_version(void) { return 47; }
 
 int mh_launch_log(int enable) {
     std::lock_guard<std::mutex> lock(g_log_mu);
@@ -921,11 +921,11 @@ int mh_mlp_fwd_ws(mh_module* m, const float* ef, const float* WhT, const uint16_
 }
 
 int mh_mlp_tangents(mh_module* m, const float* ef, const float* dfeats, const float* WhT, float* t3, int64_t E,
-                    const int32_t* rows, const int32_t* count, int32_t byrow, void* stream) {
+                    const int32_t* rows, const int32_t* count, void* stream) {
     if (E > 0 && (!ef || !dfeats || !WhT || !t3)) return fail(-1, "mh_mlp_tangents: NULL operand");
     if ((rows == nullptr) != (count == nullptr)) return fail(-1, "mh_mlp_tangents: rows and count go together");
     if (E <= 0) return 0;
-    void* args[] = {&ef, &dfeats, &WhT, &t3, &E, &rows, &count, &byrow};
+    void* args[] = {&ef, &dfeats, &WhT, &t3, &E, &rows, &count};
     return launch(m, MH_MLP_H3T, E, args, stream, "mh_mlp_tangents");
 }
 

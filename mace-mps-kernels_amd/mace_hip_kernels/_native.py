@@ -30,7 +30,7 @@ MH_CONV_FWD, MH_CONV_BWD, MH_CONV_BWD_WY, MH_SC_FWD, MH_SC_BWD, MH_CONV_BWD_R, M
     MH_EDGE_BWD, MH_MLP_BWD_P, MH_LIN_BWD_SUM, MH_MLP_H3T, MH_CONV_BWD_T, \
     MH_GEOM_STRAIN, MH_GEOM_DET, MH_MLP_BWD_W = range(84)
 MH_WANT_GX, MH_WANT_GWY, MH_CUT_MASKED, MH_CUT_NOZERO = 1, 2, 4, 8
-ABI_VERSION = 46
+ABI_VERSION = 47
 
 # hipcc/hipRTC options for every generated layer: gfx950 code, -O3, and packed-FP32 instructions disabled.
 ARCH = os.environ.get('MACE_HIP_ARCH', 'gfx950')
@@ -87,7 +87,7 @@ _SIGS = {
     'mh_edge_bwd2': (ctypes.c_int, [_P] * 11 + [ctypes.c_int64, _P]),
     'mh_edge_fwd_tan': (ctypes.c_int, [_P] * 12 + [ctypes.c_int64, _P]),
     'mh_edge_bwd_len': (ctypes.c_int, [_P] * 13 + [ctypes.c_int64, _P]),
-    'mh_mlp_tangents': (ctypes.c_int, [_P] * 5 + [ctypes.c_int64, _P, _P, _I, _P]),
+    'mh_mlp_tangents': (ctypes.c_int, [_P] * 5 + [ctypes.c_int64, _P, _P, _P]),
     'mh_mlp_out': (ctypes.c_int, [_P] * 4 + [ctypes.c_int64, _P, _P, _I, _P]),
     'mh_conv_bwd_len': (ctypes.c_int, [_P] * 18 + [_I, _I, _P]),
     'mh_perm_fwd': (ctypes.c_int, [_P] * 3 + [ctypes.c_int, _P]),

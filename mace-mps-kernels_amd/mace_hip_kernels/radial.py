@@ -791,17 +791,16 @@ def _source(spec, second):
 
     def h3t_kernel(name):
         """mlp_h3t: the derivative of ``mlp_h3``'s result in the edge length (the hidden layers on dual numbers, the
-        features ef carrying their derivatives dfe): slot i < count (edge rows[i]) stores dh/dr to ``t3`` at row i, or
-        with ``byrow`` at row rows[i].  The output layer over it gives the derivatives of the W0 rows."""
+        features ef carrying their derivatives dfe): slot i < count (edge rows[i]) stores dh/dr to ``t3`` at row i.
+        The output layer over it gives the derivatives of the W0 rows."""
         H = head(name, 'const float* __restrict__ ef, const float* __restrict__ dfe, const float* __restrict__ Wh, '
-                 'float* __restrict__ t3, long long E', Lo['tr_size'], 1, indexed=True, extra=', int byrow')
+                 'float* __restrict__ t3, long long E', Lo['tr_size'], 1, indexed=True)
         H += skip_block(1, zero_rows=False)
         H += xin(range(1)) + xin(range(1), 'dfe', 'xv')
         H += stage('Wh', Lo['tr_size']) + ['  __syncthreads();']
         H += hidden_fwd(True, False, range(1), dual=True, keep_t=True)
-        H += ['  if (do0) {',
-              f'    const long long at = (byrow ? rowc0 : ej0) * {HL};']
-        H += [f'    *reinterpret_cast<mh_f4*>(t3 + at + {32 * st + 4 * tt} + 8 * q) = ht{nh - 1}_0[{2 * st + tt}];'
+        H += ['  if (do0) {']
+        H += [f'    *reinterpret_cast<mh_f4*>(t3 + ej0 * {HL} + {32 * st + 4 * tt} + 8 * q) = ht{nh - 1}_0[{2 * st + tt}];'
               for st in range(S) for tt in range(2)]
         H += ['  }', '}', '']
         return H
@@ -1078,14 +1077,14 @@ def mlp_forward(op, ef, rows=None, count=None):
     return out
 
 
-def mlp_tangents(op, ef, dfeats, rows, count, byrow=False):
+def mlp_tangents(op, ef, dfeats, rows, count):
     """dh/dr [E, 64]: the derivative of the listed rows' last hidden activations in the edge length, from the features
-    and their derivatives in it (``mlp_h3t``); at slot i for edge rows[i], or with ``byrow`` at row rows[i]."""
+    and their derivatives in it (``mlp_h3t``); at slot i for edge rows[i]."""
     E = ef.shape[0]
     t3 = torch.empty(E, op.spec.hs[-2], device=ef.device, dtype=torch.float32)
     P = _native.ptr
     _native.launch(f'mlp_tangents[{op.tag}]', _native.load().mh_mlp_tangents, op.module.handle, P(ef), P(dfeats), P(op.WhT),
-                   P(t3), E, P(rows), P(count), int(byrow), _native.stream_of(ef))
+                   P(t3), E, P(rows), P(count), _native.stream_of(ef))
     return t3
 
 

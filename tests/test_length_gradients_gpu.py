@@ -32,14 +32,13 @@ def _close(got, want, tol):
     assert d < tol, d
 
 
-@pytest.mark.parametrize('hidden,lmax,E,byrow', [('128x0e+128x1o', 3, 1, False), ('128x0e+128x1o', 3, 1003, True),
-                                                 ('32x0e+32x1o', 2, 130, False)])
-def test_tangent_rows(hidden, lmax, E, byrow):
+@pytest.mark.parametrize('hidden,lmax,E', [('128x0e+128x1o', 3, 1), ('128x0e+128x1o', 3, 1003), ('32x0e+32x1o', 2, 130)])
+def test_tangent_rows(hidden, lmax, E):
     """mh_mlp_tangents and mh_mlp_out over a row list: rows of dW0/dr against the module in float64 (by forward-mode
     autograd).  float32 sums of 64 terms through four layers, the wide one at the accuracy of an fp32 product: 5e-6
     of the largest value."""
     dev = torch.device('cuda:0')
-    print(f'[case] tangent rows {hidden} E={E} byrow={byrow}', flush=True)
+    print(f'[case] tangent rows {hidden} E={E}', flush=True)
     model = factory.make_model(hidden, lmax, 2, elements=factory.ELEMENTS_PTCOH)
     mod, emb = model.interactions[1].conv_tp_weights, model.radial_embedding
     op = HipRadialMLP(mod, device=dev)
@@ -57,8 +56,6 @@ def test_tangent_rows(hidden, lmax, E, byrow):
     count = torch.tensor([k], dtype=torch.int32, device=dev)
     f, df = f.float().contiguous(), df.float().contiguous()
     t3 = radial.mlp_tangents(op, f, df, rows, count)
-    if byrow:                                        # the same values at the rows' own places
-        assert torch.equal(radial.mlp_tangents(op, f, df, rows, count, True)[listed], t3[:k])
     _close(radial.mlp_rows(op, t3, rows, count)[listed], dW[listed], 5e-6)
 
 
