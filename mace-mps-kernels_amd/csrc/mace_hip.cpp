@@ -307,21 +307,26 @@ int mlp_out_launch(mh_module* m, const float* h, const uint16_t* Wo, float* W, i
 // Whether the convolution forward over N receivers runs in its grouped form (four wave groups per receiver, each a
 // quarter of its edges): where that is bound and its workgroups do not fill the device more than 1.6 times over.  A
 // receiver's edges are one serial chain in the plain form, so few receivers leave the chip idle; many receivers fill
-// it and the grouped form's LDS sums only cost.  Measured (us, plain / grouped; resident workgroups 512 for the
-// 1280-weight layer, 256 for the 2176-weight one, 1,024 for the 512-weight one): 1280 weights N = 108 31.4 / 13.5, 400
-// 34.2 / 20.9, 720 41.8 / 36.8, 1176 53.4 / 58.2; 2176 weights N = 108 59.8 / 26.6, 400 65.4 / 53.0, 720 79.8 / 81.5;
-// 512 weights N = 108 11.9 / 8.7, 1176 31.9 / 24.0, 2048 36.9 / 40.3.
+// it and the grouped form's LDS sums only cost.  Measured (us, plain / grouped, 26 edges a receiver, rows in the caches;
+// resident workgroups 512 for the 1280-weight layer, 256 for the 2176-weight one, 1,024 for the 512-weight one): 1280
+// weights N = 108 26.2 / 14.0, 400 29.1 / 20.5, 720 32.2 / 32.4, 1000 38.4 / 42.8, 1176 44 / 50; 2176 weights N = 108
+// 45.0 / 22.7, 400 50.5 / 42.7, 720 60 / 71; 512 weights N = 108 12.5 / 8.5, 1176 24.5 / 20.8, 2048 30.8 / 32.1, 3600
+// 48.5 / 52.5.
 bool fwd_grouped(const mh_module* m, int kind, int64_t N) {
     return m && m->k[kind].groups > 1 && 5 * N <= 8 * m->k[kind].resident;
 }
 
 // Workgroups per receiver of the receiver-ordered backward (each takes a slice of the receiver's edges, whose outputs
 // are per edge; each loads the receiver's g row again).  By the waves that one workgroup per receiver would make,
-// against 1,024 SIMDs.  Measured (us, 1 / 2 / 4 / 8 per receiver): 1280 weights (two waves) N = 108 56.8 / 31.3 / 19.7
-// / 16.0, 400 63.0 / 43.5 / 47.4 / 40.6, 1176 120 / 117 / 115 / 114, 2048 215 / 191 / 192 / 198, 3600 339 / 321 / 326 /
-// 342, 7056 618 / 614 / 626 / 658; 2176 weights N = 1176 258 / 211 / 201 / 214, 3600 576 / 577 / 586 / 625; 512 weights
-// N = 108 28.1 / 16.2 / 11.1 / 8.5, 2048 79 / 70 / 70 / 77, 7056 283 / 297 / 286 / 297; 96 weights (one wave) N = 1176
-// 39.9 / 25.0 / 17.8 / 19.6, 7056 112 / 94 / 97 / 103.
+// against 1,024 SIMDs.  Measured (us, 1 / 2 / 4 / 8 per receiver, the dX sum included, bulk of 31 to 35 edges a receiver,
+// caches flushed between launches; runs of one shape differ by 2 to 6%): 1280 weights (two waves) N = 192 75.8 / 49.0 /
+// 36.8 / 33.5, 300 80.6 / 53.3 / 43.5 / 47.2, 400 83.3 / 60.2 / 61.7 / 55.6, 500 90.9 / 66.6 / 73.8 / 70.1, 720 105 / 92.5 /
+// 92.8 / 95.7, 1000 126 / 134 / 123 / 130, 1500 174 / 171 / 172 / 179, 2048 253 / 234 / 233 / 243, 3600 411 / 407 / 412 /
+// 429; 2176 weights N = 192 127 / 75.7 / 54.5 / 60.7, 720 184 / 186 / 167 / 179, 1500 362 / 317 / 322 / 341; 512 weights
+// N = 192 46.9 / 33.5 / 26.0 / 22.9, 720 58.0 / 44.5 / 46.5 / 45.7, 2048 94.4 / 96.9 / 97.6 / 101; 96 weights (one wave)
+// N = 384 48.9 / 32.4 / 24.5 / 20.5, 1176 55.1 / 37.5 / 30.7 / 32.7, 3072 67.1 / 65.5 / 60.2 / 61.3, 4096 76.9 / 75.4 /
+// 75.5 / 77.5.  The counts' own lines differ by layer (how the workgroups divide over the compute units): four per receiver
+// are up to 11% off the best split at 800 to 1,000 waves of the 1280-weight layer and the best or within 5% elsewhere.
 int bwd_parts(const mh_module* m, int kind, int64_t N) {
     if (!m) return 1;
     const int64_t waves = N * (m->k[kind].block / 64);
@@ -329,10 +334,13 @@ int bwd_parts(const mh_module* m, int kind, int64_t N) {
 }
 
 // The same for the backward to the lengths, whose rows two receivers share: more slices spread the two readers of a row
-// further apart in time, and with enough receivers to fill the device its caches matter more.  Measured in the model,
-// 1280 weights (us, 1 / 2 / 4 per receiver; slabs of about 160 atoms, and bulk): N = 648 98 / 72 / 74, 1626 169 / 159 / 152,
-// 2600 243 / 271 / 273, 3704 339 / 401 / 438, 5100 448 / 548 / 600; bulk 1372 157 / 158 / 160, 4000 498 / 536 / 580, 6912
-// 845 / 924 / 999 (non-temporal loads of the rows, one per receiver: 2600 242, 3704 370, 6912 951).
+// further apart in time, and with enough receivers to fill the device its caches matter more.  Measured as above, 1280
+// weights (us, 1 / 2 / 4 / 8 per receiver): N = 192 74.7 / 48.2 / 37.4 / 36.2, 300 79.5 / 54.6 / 48.7 / 49.4, 720 111 / 101
+// / 104 / 104, 1372 181 / 179 / 179 / 184, 1500 186 / 189 / 193 / 197, 1626 223 / 209 / 206 / 212, 2048 250 / 247 / 252 /
+// 257, 2600 303 / 320 / 329 / 320, 3600 408 / 436 / 458 / 453; slabs of 160 atoms: 640 93.7 / 77.0 / 76.9 / 77.0, 1600 190
+// / 175 / 172 / 178, 2080 214 / 213 / 214 / 222, 2560 236 / 258 / 258 / 261.  From 2,500 to 4,096 waves the four differ by
+// what runs of one shape do (2176 weights: N = 1500 367 / 331 / 353 / 359).  In the model, one per receiver: bulk of 6,912
+// atoms 845, with non-temporal loads of the rows 951.
 int bwd_len_parts(const mh_module* m, int kind, int64_t N) {
     if (!m) return 1;
     const int64_t waves = N * (m->k[kind].block / 64);
