@@ -42,7 +42,8 @@ from . import conv as _conv
 
 BLOCK = 256
 SEG_BLOCK = 1024          # threads of a segmented sum of 3x3 rows
-SLICE_ROWS = 8192         # edges of a structure per workgroup of that sum (8 per thread), up to MAX_SLICES workgroups
+SLICE_ROWS = 8192         # edges per workgroup of that sum, at most, for a structure of the batch's mean size (8 per
+                          # thread; a larger structure has more), while that takes no more than MAX_SLICES workgroups
 MAX_SLICES = 64
 _ACTIVE = contextvars.ContextVar('mace_hip_kernels_geometry', default=False)
 _PTR = contextvars.ContextVar('mace_hip_kernels_geometry_ptr', default=None)   # the batch's ptr during a forward
