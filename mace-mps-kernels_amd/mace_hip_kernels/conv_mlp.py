@@ -784,6 +784,14 @@ class ConvRadialFn(torch.autograd.Function):
         return gx, gY, glen
 
 
+def takes_lengths(conv):
+    """Whether ``conv`` is a convolution whose backward can go to the edge lengths: its radial MLP inside its own node
+    and covered by the weight-stationary output kernel."""
+    from .conv import HipConvTP
+    mlp = conv.deferred_mlp() if isinstance(conv, HipConvTP) else None
+    return mlp is not None and mlp.spec.hs[-2] == 64
+
+
 def length_tangents(w, mlp):
     """(lengths alias, (dfeats, dcutoff, the lengths' grad_fn, Watch)) for ``ConvRadialFn`` on the unformed weights ``w``
     (a ``FusedWeights`` of ``mlp``), or nothing where its gradient to the lengths does not apply: fewer edges than the row

@@ -360,8 +360,9 @@ class _GeomFn(torch.autograd.Function):
             # derivatives in the length only where a convolution may take them (conv_mlp.length_tangents: not with a
             # gradient of the shifts, as stress has, and not for a double backward)
             from . import edgefeat
-            edgefeat.forward_all(p, gr, sh, vec, ln, edge_ops,
-                                 tangents=ctx.needs_input_grad[0] and not ctx.needs_input_grad[1]
+            *ops, lengths = edge_ops
+            edgefeat.forward_all(p, gr, sh, vec, ln, ops,
+                                 tangents=lengths and ctx.needs_input_grad[0] and not ctx.needs_input_grad[1]
                                  and not double_backward and _conv.PAIR_GRADS and _conv.LENGTH_GRADS
                                  and E >= _conv.EDGE_COMPACT_MIN)
         else:
@@ -725,13 +726,15 @@ def _wrap_scatter(orig):
 
 
 def _edge_ops(model):
-    """(harmonics, embedding) of ``model`` when both are drop-ins and the fused edge pass is on, else None."""
+    """(harmonics, embedding, whether a convolution can take the gradient to the edge lengths) of ``model`` when the two
+    are drop-ins and the fused edge pass is on, else None."""
     from . import edgefeat
+    from .conv_mlp import takes_lengths
     from .edge import HipSphericalHarmonics
     from .embedding import HipRadialEmbedding
     sh, emb = getattr(model, 'spherical_harmonics', None), getattr(model, 'radial_embedding', None)
     if edgefeat.FUSE and isinstance(sh, HipSphericalHarmonics) and isinstance(emb, HipRadialEmbedding):
-        return sh, emb
+        return sh, emb, any(takes_lengths(getattr(b, 'conv_tp', None)) for b in getattr(model, 'interactions', ()))
     return None
 
 

@@ -267,6 +267,17 @@ def test_captured_replays(models):
         assert torch.equal(got['forces'], want['forces']) and torch.equal(got['energy'], want['energy'])
 
 
+def test_which_models_form_derivatives(models, monkeypatch):
+    """Only a model with a convolution that takes the gradient to the lengths: its radial MLP inside its node."""
+    from mace_hip_kernels import geometry
+    _, met = models
+    print('[case] models that form derivatives', flush=True)
+    assert geometry._edge_ops(met)[2]
+    for blk in met.interactions:
+        monkeypatch.setattr(blk.conv_tp, '_deferred_mlp', None)
+    assert not geometry._edge_ops(met)[2]
+
+
 def test_second_layer_energy_only(models):
     """No gradients wanted: neither tangents nor their rows are formed, energies as with them."""
     _, met = models
