@@ -59,7 +59,8 @@ def test_tangent_rows(hidden, lmax, E):
     _close(radial.mlp_rows(op, t3, rows, count)[listed], dW[listed], 5e-6)
 
 
-@pytest.mark.parametrize('hidden,n,want_x', [('128x0e+128x1o', 41, True), ('128x0e', 900, False),
+# (8, 4, 1, 4 and 8 workgroups per receiver)
+@pytest.mark.parametrize('hidden,n,want_x', [('128x0e+128x1o', 41, True), ('128x0e', 900, False), ('128x0e', 2049, True),
                                              ('96x0e+96x1o', 200, True), ('128x0e+128x1o+128x2e', 60, True)])
 def test_backward_to_the_lengths(hidden, n, want_x):
     """mh_conv_bwd_len on rows read through a map, with edges outside the cutoff's support, against the plain
