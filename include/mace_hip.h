@@ -169,10 +169,11 @@ int mh_module_bind(mh_module* m, int kind, const char* name, int block_threads, 
 /* As mh_module_bind, with a second grid dimension of grid_y workgroups (1..65535); mh_module_bind uses 1. */
 int mh_module_bind_grid(mh_module* m, int kind, const char* name, int block_threads, int rows_per_block,
                         int grid_y);
-/* The kernel bound to `kind` may also be launched with groups x block_threads threads and lds_bytes of dynamic LDS
- * (the convolution forwards: conv_codegen.fwd_groups and fwd_groups_lds give both), in which `groups` wave groups
- * share each row; the entry points choose that form for small launches.  Without this call they never do. */
-int mh_module_bind_groups(mh_module* m, int kind, int groups, int lds_bytes);
+/* Attach kernel `name` to slot `kind` (bound already) as its form for few rows, with the same parameters and launched
+ * with groups x block_threads threads and lds_bytes of dynamic LDS (the convolution forwards: conv_codegen.fwd_groups
+ * and fwd_groups_lds give both): `groups` wave groups share each row.  The entry points choose it for small launches;
+ * without this call they never do.  The launch log names the slot's own symbol for either form. */
+int mh_module_bind_groups(mh_module* m, int kind, const char* name, int groups, int lds_bytes);
 
 /* Fused convolution forward: out[n] = Σ_{p in rowptr[n]..rowptr[n+1]} TP(x[senders[e]], Y[e], W[e]), e = eids[p].
  * rowptr/eids: receiver-sorted CSR.  Replaces lib.conv_fwd (reference conv.py:109-141, launched at conv.py:247). */

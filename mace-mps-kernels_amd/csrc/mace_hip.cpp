@@ -37,8 +37,9 @@ struct Kernel {
     int block = 0;
     int rows_per_block = 1;
     int grid_y = 1;          // second grid dimension (a fixed count: output blocks of a node linear)
-    int groups = 1;          // the kernel also runs with groups x block threads and `lds` bytes of dynamic LDS
-    int lds = 0;             // (mh_module_bind_groups), of which `resident` workgroups fit on the device at once
+    hipFunction_t gfn = nullptr;   // its form for few rows (mh_module_bind_groups): groups x block threads and `lds`
+    int groups = 1;                // bytes of dynamic LDS, of which `resident` workgroups fit on the device at once
+    int lds = 0;
     int64_t resident = 0;
 };
 
@@ -87,7 +88,7 @@ int launch(mh_module* m, int kind, int64_t rows, void** args, void* stream, cons
     }
     int64_t grid = (rows + k.rows_per_block - 1) / k.rows_per_block;
     if (grid > 0x7fffffffLL) return fail(-1, std::string(what) + ": launch too large");
-    hipError_t e = hipModuleLaunchKernel(k.fn, static_cast<unsigned>(grid),
+    hipError_t e = hipModuleLaunchKernel(grouped ? k.gfn : k.fn, static_cast<unsigned>(grid),
                                          static_cast<unsigned>(grid_y > 0 ? grid_y : k.grid_y), 1,
                                          static_cast<unsigned>(grouped ? k.groups * k.block : k.block), 1, 1,
                                          static_cast<unsigned>(grouped ? k.lds : 0), static_cast<hipStream_t>(stream),
@@ -146,7 +147,7 @@ extern "C" {
 
 const char* mh_last_error(void) { return g_err.c_str(); }
 
-int mh_version(void) { return 47; }
+int mh_version(void) { return 48; }
 
 int mh_launch_log(int enable) {
     std::lock_guard<std::mutex> lock(g_log_mu);
@@ -259,23 +260,27 @@ int mh_module_bind_grid(mh_module* m, int kind, const char* name, int block_thre
     m->k[kind].block = block_threads;
     m->k[kind].rows_per_block = rows_per_block;
     m->k[kind].grid_y = grid_y;
+    m->k[kind].gfn = nullptr;
     m->k[kind].groups = 1;
     return 0;
 }
 
-int mh_module_bind_groups(mh_module* m, int kind, int groups, int lds_bytes) {
-    if (!m) return fail(-1, "mh_module_bind_groups: null argument");
+int mh_module_bind_groups(mh_module* m, int kind, const char* name, int groups, int lds_bytes) {
+    if (!m || !name) return fail(-1, "mh_module_bind_groups: null argument");
     if (kind < 0 || kind >= MH_NUM_KINDS || !m->k[kind].fn) return fail(-1, "mh_module_bind_groups: kind not bound");
     Kernel& k = m->k[kind];
     if (groups < 2 || groups * k.block > 1024 || lds_bytes < 0)
         return fail(-1, "mh_module_bind_groups: bad launch shape");
-    MH_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k.fn), hipFuncAttributeMaxDynamicSharedMemorySize,
+    hipFunction_t fn = nullptr;
+    MH_HIP(hipModuleGetFunction(&fn, m->mod, name));
+    MH_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize,
                                lds_bytes));
     int per_cu = 0, cus = 0;
-    MH_HIP(hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k.fn, groups * k.block,
+    MH_HIP(hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, groups * k.block,
                                                               static_cast<size_t>(lds_bytes)));
     MH_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, m->device));
     if (per_cu < 1) return fail(-1, "mh_module_bind_groups: the grouped workgroup does not fit");
+    k.gfn = fn;
     k.groups = groups;
     k.lds = lds_bytes;
     k.resident = static_cast<int64_t>(per_cu) * cus;
@@ -313,7 +318,7 @@ int mlp_out_launch(mh_module* m, const float* h, const uint16_t* Wo, float* W, i
 // 45.0 / 22.7, 400 50.5 / 42.7, 720 60 / 71; 512 weights N = 108 12.5 / 8.5, 1176 24.5 / 20.8, 2048 30.8 / 32.1, 3600
 // 48.5 / 52.5.
 bool fwd_grouped(const mh_module* m, int kind, int64_t N) {
-    return m && m->k[kind].groups > 1 && 5 * N <= 8 * m->k[kind].resident;
+    return m && m->k[kind].gfn && 5 * N <= 8 * m->k[kind].resident;
 }
 
 // Workgroups per receiver of the receiver-ordered backward (each takes a slice of the receiver's edges, whose outputs

@@ -30,7 +30,7 @@ MH_CONV_FWD, MH_CONV_BWD, MH_CONV_BWD_WY, MH_SC_FWD, MH_SC_BWD, MH_CONV_BWD_R, M
     MH_EDGE_BWD, MH_MLP_BWD_P, MH_LIN_BWD_SUM, MH_MLP_H3T, MH_CONV_BWD_T, \
     MH_GEOM_STRAIN, MH_GEOM_DET, MH_MLP_BWD_W = range(84)
 MH_WANT_GX, MH_WANT_GWY, MH_CUT_MASKED, MH_CUT_NOZERO = 1, 2, 4, 8
-ABI_VERSION = 47
+ABI_VERSION = 48
 
 # hipcc/hipRTC options for every generated layer: gfx950 code, -O3, and packed-FP32 instructions disabled.
 ARCH = os.environ.get('MACE_HIP_ARCH', 'gfx950')
@@ -51,7 +51,7 @@ _SIGS = {
     'mh_module_load': (ctypes.c_int, [_P, ctypes.c_size_t, ctypes.POINTER(_P)]),
     'mh_module_unload': (ctypes.c_int, [_P]),
     'mh_module_bind': (ctypes.c_int, [_P, ctypes.c_int, ctypes.c_char_p, ctypes.c_int, ctypes.c_int]),
-    'mh_module_bind_groups': (ctypes.c_int, [_P, ctypes.c_int, ctypes.c_int, ctypes.c_int]),
+    'mh_module_bind_groups': (ctypes.c_int, [_P, ctypes.c_int, ctypes.c_char_p, ctypes.c_int, ctypes.c_int]),
     'mh_conv_fwd': (ctypes.c_int, [_P] * 8 + [_I, _P]),
     'mh_conv_bwd_x': (ctypes.c_int, [_P] * 8 + [_I, _P]),
     'mh_conv_bwd_wy': (ctypes.c_int, [_P] * 9 + [_I, _P]),
@@ -214,10 +214,11 @@ class Module:
             check(lib.mh_module_bind_grid(self.handle, kind, name.encode(), block, rows, grid_y[0] if grid_y else 1),
                   f'bind {name}')
 
-    def bind_groups(self, kinds, groups, lds):
-        """Let the kernels bound to ``kinds`` also run as ``groups`` wave groups per row (``mh_module_bind_groups``)."""
-        for kind in kinds:
-            check(self._lib.mh_module_bind_groups(self.handle, kind, groups, lds), 'bind groups')
+    def bind_groups(self, kernels, groups, lds):
+        """Bind ``kernels`` {slot: symbol} as the slots' forms with ``groups`` wave groups per row
+        (``mh_module_bind_groups``)."""
+        for kind, name in kernels.items():
+            check(self._lib.mh_module_bind_groups(self.handle, kind, name.encode(), groups, lds), f'bind {name}')
 
     def __del__(self):
         h = getattr(self, 'handle', None)

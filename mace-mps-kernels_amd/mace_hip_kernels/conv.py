@@ -1054,7 +1054,9 @@ class HipConvTP(torch.nn.Module):
             })
             groups = fwd_groups(self.spec)
             if groups:
-                self.module.bind_groups((_native.MH_CONV_FWD, _native.MH_CONV_FWD_C, _native.MH_CONV_FWD_CR), groups,
+                self.module.bind_groups({_native.MH_CONV_FWD: self.spec.kname('conv_fwdg'),
+                                         _native.MH_CONV_FWD_C: self.spec.kname('conv_fwdcg'),
+                                         _native.MH_CONV_FWD_CR: self.spec.kname('conv_fwdcrg')}, groups,
                                         fwd_groups_lds(self.spec))
         self.irreps_in1, self.irreps_in2, self.irreps_out = tp.irreps_in1, tp.irreps_in2, tp.irreps_out
         self.instructions = tp.instructions

@@ -80,7 +80,7 @@ GY_LDS_ATOMIC = True
 CHUNK_LDS = 24576
 
 
-# Forward with few receivers: launched with FWD_GROUPS x BLOCK threads, FWD_GROUPS wave groups share a receiver, each
+# Forward with few receivers (conv_fwd*g): FWD_GROUPS wave groups of one workgroup share a receiver, each
 # walking its own slice of the receiver's edges (in chunks of CHUNK / FWD_GROUPS), and their partial sums are added in
 # LDS in a fixed order.  A receiver's edges are one serial chain of about 1 us each, so with fewer workgroups than the
 # chip holds the chain is the kernel's time; FWD_GROUPS slices cut it to a quarter.
@@ -293,9 +293,8 @@ def chunk_edges(npp):
 
 
 def fwd_groups(spec):
-    """Wave groups per receiver of the forward kernels' few-receivers form, 0 where it does not fit: 512 threads (so
-    that the larger launch leaves the registers of the smaller one alone), and the partial sums beside the coupling
-    products within a compute unit's LDS."""
+    """Wave groups per receiver of the forward's few-receivers kernels, 0 where there are none: at most 512 threads (256
+    registers each), and the partial sums beside the coupling products within a compute unit's LDS."""
     npp = (len({(co['k'], a, c) for co in spec.coef for a, _, c, _ in co['terms']}) + 3) // 4 * 4
     lds = fwd_groups_lds(spec) + 4 * chunk_edges(npp) * (npp + spec.ncb)
     return FWD_GROUPS if FWD_GROUPS * spec.block <= 512 and lds <= 153600 else 0
@@ -356,22 +355,20 @@ def source(spec):
     ms_decl_c = ['  __shared__ float4 Ms4[CHUNK][NPP / 4];',
                  '  float (*Ms)[NPP] = reinterpret_cast<float (*)[NPP]>(Ms4);']
     # ------------------------------------------------------------------------------------------- forward
-    def fwd_kernel(cut, rows=False):
+    def fwd_kernel(cut, rows=False, groups=1):
         """``cut`` (kernel ``conv_fwdc``): the weights are W0·c with a per-edge scalar c, read as W0 and scaled in
         registers (the product is never formed in memory); an edge with c == 0 (padding, or past r_max in a
         neighbour list with a skin) contributes exactly zero, so each chunk of 64 edges is first compacted to its
         edges with c != 0 (ballot, then a per-wave LDS scatter by lane rank) and only those are walked.  Every wave
         of the workgroup builds the same list, so the barriers stay uniform.
 
-        A workgroup of BLOCK threads walks a receiver's edges itself; one of ``fwd_groups`` x BLOCK threads (with
-        ``fwd_groups_lds`` bytes of dynamic LDS) as that many wave groups, each a slice of them."""
-        groups = fwd_groups(spec)
-        # the two forms' registers together: held to three waves per SIMD (the plain form's own count; 184 VGPRs and
-        # two waves for the 2176-weight layer otherwise) where the accumulators and prefetches leave room for it
-        occ = '__attribute__((amdgpu_waves_per_eu(3))) ' if groups and no + 2 * (nx + nk) <= 130 else ''
+        ``groups`` > 1 (kernels ``conv_fwd*g``, launched with ``fwd_groups_lds`` bytes of dynamic LDS): ``groups`` wave
+        groups share a receiver, each a slice of its edges.  Kernels of their own: as a second body of the plain ones
+        they raised those by 6 to 30 registers (64-channel l_max 3 layer, 4,000 receivers, factored 260 us to 268)."""
+        base = ('conv_fwdcr' if rows else 'conv_fwdc') if cut else 'conv_fwd'
         F = [
-            f'extern "C" __global__ __launch_bounds__({max(1, groups)} * BLOCK) {occ}void '
-            f'{spec.kname(("conv_fwdcr" if rows else "conv_fwdc") if cut else "conv_fwd")}(',
+            f'extern "C" __global__ __launch_bounds__({f"{groups} * " if groups > 1 else ""}BLOCK) void '
+            f'{spec.kname(base + ("g" if groups > 1 else ""))}(',
             '    const float* __restrict__ x, const float* __restrict__ Y, const float* __restrict__ W,',
             '    const int* __restrict__ rowptr, const int* __restrict__ eids, const int* __restrict__ senders,',
             '    float* __restrict__ out, int N' + (', const float* __restrict__ cutv, const int* __restrict__ wrow) {'
@@ -380,12 +377,7 @@ def source(spec):
             '  const int n = mh_xcd_block(blockIdx.x, gridDim.x);',
             '  if (n >= N) return;',
         ]
-        if groups:
-            F += ['  if (blockDim.x == BLOCK) {'] + ['  ' + t for t in fwd_walk(cut, rows, 1)] + ['  } else {']
-            F += ['  ' + t for t in fwd_walk(cut, rows, groups)] + ['  }']
-        else:
-            F += fwd_walk(cut, rows, 1)
-        return F + ['}', '']
+        return F + fwd_walk(cut, rows, groups) + ['}', '']
 
     def fwd_walk(cut, rows, groups):
         """The body of a forward kernel for ``groups`` wave groups per receiver: group i walks the i-th slice of the
@@ -479,6 +471,9 @@ def source(spec):
         return F + ['  }']
 
     L += fwd_kernel(False) + fwd_kernel(True) + fwd_kernel(True, rows=True)
+    if fwd_groups(spec):
+        L += (fwd_kernel(False, groups=FWD_GROUPS) + fwd_kernel(True, groups=FWD_GROUPS)
+              + fwd_kernel(True, rows=True, groups=FWD_GROUPS))
     # ----------------------------------------------------------------------------------- fused backward
     L += [
         f'extern "C" __global__ __launch_bounds__(BLOCK) void {spec.kname("conv_bwd")}(',

@@ -672,10 +672,10 @@ class ConvRadialFn(torch.autograd.Function):
 
     With a lengths alias ``ln`` and ``tan`` = (dfeats/dr, dcutoff/dr, the lengths' grad_fn, a Watch)
     (``length_tangents``) the gradient goes to the lengths instead of to ef and cut: the weights are a function
-    W0(r) c(r) of each edge's length, so dL/dr[e] = sum_k,u dL/d(W0 c)[e, k, u] (c dW0/dr + c' W0), which the convolution's backward reduces in registers
-    (``conv_bwdt``) against rows of dW0/dr, formed from the hidden layers' derivatives in r by the forward's output
-    kernel, one row per edge and its reverse.  dL/dW0 is neither stored nor projected (1280 weights, 78k edges of 39k
-    rows: the projection's 140 us become 27 + 55).  A backward that may want the gradients of ef or cut themselves (the
+    W0(r) c(r) of each edge's length, so dL/dr[e] = sum_k,u dL/d(W0 c)[e, k, u] (c dW0/dr + c' W0), which the
+    convolution's backward reduces in registers (``conv_bwdt``) against rows of dW0/dr, formed from the hidden layers'
+    derivatives in r by the forward's output kernel, one row per edge and its reverse.  dL/dW0 is neither stored nor
+    projected (1280 weights, 78k edges of 39k rows: the projection's 140 us become 27 + 55).  A backward that may want the gradients of ef or cut themselves (the
     lengths' own producer not run by it, or ``edgefeat.Watch.wanted``) takes the form above.  No double
     backward: the two-kernel modules take that (``patch_model(double_backward=True)``)."""
 

@@ -1,5 +1,6 @@
 """
-The generated convolution source under its prefetch knob: every kernel either follows the knob or ignores it whole.
+The generated convolution source: its prefetch knob, which every kernel either follows or ignores whole, and the kernels of
+the forward over few receivers.
 """
 import re
 
@@ -35,3 +36,17 @@ def test_backward_prefetch_reloads_every_row_it_reads(monkeypatch, hidden):
     for base in ('conv_bwdr', 'conv_bwdrc'):
         k = two[spec.kname(base)]
         assert k != one[spec.kname(base)] and 'wn0 = wm0;' in k and 'xn0 = xm0;' in k
+
+
+@pytest.mark.parametrize('hidden,grouped', [('128x0e+128x1o', True), ('32x0e+32x1o', True), ('192x0e', False)])
+def test_few_receivers_have_kernels_of_their_own(hidden, grouped):
+    """The wave groups' body in the plain kernels would cost every launch its registers."""
+    spec = _spec(hidden, 2)
+    assert bool(conv_codegen.fwd_groups(spec)) == grouped
+    k = _kernels(conv_codegen.source(spec))
+    for base in ('conv_fwd', 'conv_fwdc', 'conv_fwdcr'):
+        plain, few = k[spec.kname(base)], k.get(spec.kname(base + 'g'))
+        assert '__launch_bounds__(BLOCK)' in plain and 'red_[]' not in plain and 'grp' not in plain
+        assert (few is not None) == grouped
+        if grouped:
+            assert '__launch_bounds__(4 * BLOCK)' in few and 'red_[]' in few
