@@ -356,15 +356,10 @@ class _GeomFn(torch.autograd.Function):
         vec = torch.empty(E, 3, device=p.device, dtype=torch.float32)
         ln = torch.empty(E, 1, device=p.device, dtype=torch.float32)
         if edge_ops is not None:
-            # the harmonics and the embedding of the same edges in the same pass, left on vec for those modules; the
-            # derivatives in the length only where a convolution may take them (conv_mlp.length_tangents: not with a
-            # gradient of the shifts, as stress has, and not for a double backward)
+            # the harmonics and the embedding of the same edges in the same pass, left on vec for those modules
             from . import edgefeat
-            *ops, lengths = edge_ops
-            edgefeat.forward_all(p, gr, sh, vec, ln, ops,
-                                 tangents=lengths and ctx.needs_input_grad[0] and not ctx.needs_input_grad[1]
-                                 and not double_backward and _conv.PAIR_GRADS and _conv.LENGTH_GRADS
-                                 and E >= _conv.EDGE_COMPACT_MIN)
+            *ops, tangents = edge_ops
+            edgefeat.forward_all(p, gr, sh, vec, ln, ops, tangents=tangents)
         else:
             mod = _module(p.device)
             _native.launch('geom_fwd', _native.load().mh_geom_fwd, mod.handle, _native.ptr(p), _native.ptr(gr.send),
@@ -431,7 +426,10 @@ def edge_vectors_and_lengths(positions, edge_index, shifts):
     if positions.shape[-1] != 3 or shifts.shape != (edge_index.shape[1], 3):
         raise ValueError(f'positions [N, 3] and shifts [E, 3] expected, got {tuple(positions.shape)}, '
                          f'{tuple(shifts.shape)}')
-    vec, ln = _GeomFn.apply(positions, shifts, edge_index, _ACTIVE.get() == 'double_backward', _EDGE.get())
+    double_backward, ops = _ACTIVE.get() == 'double_backward', _EDGE.get()
+    if ops is not None:
+        ops = (*ops[:2], ops[2] and not double_backward and _length_gradients(positions, shifts))
+    vec, ln = _GeomFn.apply(positions, shifts, edge_index, double_backward, ops)
     if not shifts.requires_grad:
         # The lengths' one differentiable input is then the positions, through pos[recv] - pos[send] + shift: an edge
         # and its exact reverse (negated vector) have equal lengths whose gradients reach the two end atoms along the
@@ -439,6 +437,13 @@ def edge_vectors_and_lengths(positions, edge_index, shifts):
         # patched radial embedding passes this on to its features (lengths_pair_symmetric).
         ln._mh_vec = (ln._version, vec, vec._version)
     return vec, ln
+
+
+def _length_gradients(positions, shifts):
+    """Whether convolutions of these edges may take the gradient to the lengths (conv_mlp.length_tangents), and so read
+    the embedding's derivatives in them: not without gradients, nor with one of the shifts, as stress has."""
+    return (torch.is_grad_enabled() and positions.requires_grad and not shifts.requires_grad and _conv.PAIR_GRADS
+            and _conv.LENGTH_GRADS and shifts.shape[0] >= _conv.EDGE_COMPACT_MIN)
 
 
 def lengths_pair_symmetric(t):

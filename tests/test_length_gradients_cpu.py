@@ -5,24 +5,35 @@ backward can tell of a wish for the gradients it leaves out.
 """
 import pytest
 import torch
+from torch._subclasses.fake_tensor import FakeTensorMode
 
 from mace_hip_kernels import edgefeat, geometry as G
 
 
-@pytest.mark.parametrize('grad_pos,grad_shifts,double_backward,edges,takes,want', [
-    (True, False, False, 16384, True, True), (True, False, False, 16383, True, False),
-    (False, False, False, 16384, True, False), (True, True, False, 16384, True, False),
-    (True, False, True, 16384, True, False), (True, False, False, 16384, False, False)])
-def test_derivatives_are_formed_where_a_convolution_takes_them(monkeypatch, grad_pos, grad_shifts, double_backward,
-                                                               edges, takes, want):
-    """A gradient of the shifts (stress), a double backward, or radial MLPs outside the convolutions' nodes keep the
-    convolutions on the dL/dW0 form, which reads neither dfeats nor dcutoff."""
+@pytest.mark.parametrize('grad_pos,grad_shifts,active,edges,takes,grad,want', [
+    (True, False, True, 16384, True, True, True), (True, False, True, 16383, True, True, False),
+    (False, False, True, 16384, True, True, False), (True, True, True, 16384, True, True, False),
+    (True, False, 'double_backward', 16384, True, True, False), (True, False, True, 16384, False, True, False),
+    (True, False, True, 16384, True, False, False)])
+def test_derivatives_are_formed_where_a_convolution_takes_them(monkeypatch, grad_pos, grad_shifts, active, edges, takes,
+                                                               grad, want):
+    """A gradient of the shifts (stress), a double backward, radial MLPs outside the convolutions' nodes, or no gradients
+    at all (positions that require one under no_grad, as MACE's do): nothing reads dfeats and dcutoff."""
     asked = []
     monkeypatch.setattr(G._conv, 'graph_for', lambda ei, n: None)
+    monkeypatch.setattr(G, '_together', lambda *t: True)
     monkeypatch.setattr(edgefeat, 'forward_all', lambda *a, tangents=False: asked.append(bool(tangents)))
-    pos = torch.zeros(4, 3, requires_grad=grad_pos)
-    shifts = torch.zeros(edges, 3, requires_grad=grad_shifts)
-    G._GeomFn.apply(pos, shifts, torch.zeros(2, edges, dtype=torch.int64), double_backward, ('sh', 'emb', takes))
+    with FakeTensorMode(allow_non_fake_inputs=True):
+        pos = torch.zeros(4, 3, device='cuda', requires_grad=grad_pos)
+        shifts = torch.zeros(edges, 3, device='cuda', requires_grad=grad_shifts)
+        ei = torch.zeros(2, edges, device='cuda', dtype=torch.int64)
+        tokens = G._ACTIVE.set(active), G._EDGE.set(('sh', 'emb', takes))
+        try:
+            with torch.set_grad_enabled(grad):
+                G.edge_vectors_and_lengths(pos, ei, shifts)
+        finally:
+            G._EDGE.reset(tokens[1])
+            G._ACTIVE.reset(tokens[0])
     assert asked == [want]
 
 
