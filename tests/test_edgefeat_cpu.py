@@ -129,3 +129,56 @@ def test_fused_edge_kernels_equal_the_separate_ones(hidden, lmax, tmp_path):
         _call(getattr(em, 'run_' + es.kname('emb_bwd')), ln, tf, tc, wl, E=E)
         assert np.array_equal(gv.view(np.uint32), wv.view(np.uint32)), (first_cut, keep)
         assert np.array_equal(gl.view(np.uint32), wl.view(np.uint32)), (first_cut, keep)
+
+
+@pytest.mark.skipif(shutil.which('g++') is None, reason='needs g++')
+def test_forms_for_the_gradients_to_the_lengths(tmp_path):
+    """``edge_fwd`` with derivative buffers: its outputs unchanged bit for bit, and the derivatives in the length against
+    the embedding in float64 (float32 values up to w^2 ~ 40 from a few products: 2e-5).  ``edge_bwd`` with gradients of
+    the lengths: what it gives without them plus their sum, and without the features' gradients the sum alone."""
+    torch = pytest.importorskip('torch')
+    model = factory.make_model('32x0e+32x1o', 2, 2, elements=factory.ELEMENTS_PTCOH)
+    ss, es = edge.SHSpec(model.spherical_harmonics), embedding.EmbSpec(model.radial_embedding)
+    f = 'const float* a0, const int* a1, const int* a2, const float* a3, float* a4, float* a5, float* a6, float* a7, ' \
+        'float* a8'
+    b = 'const float* a0, const float* a1, const float* a2, const float* a3, const float* a4, float* a5, float* a6, ' \
+        'const float* a7, const float* a8, const float* a9'
+    fa, ba = ', '.join(f'a{i}' for i in range(9)), ', '.join(f'a{i}' for i in range(7))
+    kf, kb = edgefeat.kname(ss, es, 'edge_fwd'), edgefeat.kname(ss, es, 'edge_bwd')
+    src = edgefeat.source(ss, es)
+    lib = _library(src, {kf: (f, fa), kb: (b, ba, 'a7, a8, a9')}, tmp_path, 'plain')
+    ext = _library(src, {kf: (f + ', float* a9, float* a10', fa, 'a9, a10'),
+                         kb: (b + ', const float* a10, const float* a11', ba, 'a7, a8, a9, a10, a11')}, tmp_path, 'ext')
+    rng = np.random.default_rng(5)
+    N, E = 40, 515
+    pos = rng.uniform(0.0, 6.0, size=(N, 3)).astype(np.float32)
+    send = rng.integers(0, N, E).astype(np.int32)
+    recv = ((send + rng.integers(1, N, E)) % N).astype(np.int32)      # (no zero lengths: NaN != NaN below)
+    shifts = np.zeros((E, 3), np.float32)
+    z = lambda *a: np.zeros(a, np.float32)  # noqa: E731
+    new = lambda: [z(E, 3), z(E), z(E, ss.dim), z(E, es.n), z(E)]  # noqa: E731
+    plain, tan, df, dc = new(), new(), z(E, es.n), z(E)
+    _call(getattr(lib, 'run_' + kf), pos, send, recv, shifts, *plain, E=E)
+    _call(getattr(ext, 'run_' + kf), pos, send, recv, shifts, *tan, df, dc, E=E)
+    for a, c in zip(plain, tan):
+        assert np.array_equal(a.view(np.uint32), c.view(np.uint32))
+    ok = plain[1] > 0.3                              # (1/x amplifies the rounding of shorter ones)
+    emb = model.radial_embedding.double()
+    r = torch.tensor(plain[1][ok].astype(np.float64))[:, None]
+    _, (wf, wc) = torch.func.jvp(lambda x: tuple(emb(x)), (r,), (torch.ones_like(r),))
+    assert np.abs(df[ok] - wf.numpy()).max() < 2e-5 and np.abs(dc[ok] - wc.numpy()[:, 0]).max() < 2e-5
+    vec, ln = plain[0], plain[1]
+    gY, gf, gc, g1, g2 = (rng.normal(size=k).astype(np.float32) for k in ((E, ss.dim), (E, es.n), E, E, E))
+    out = lambda *a: _bwd(ext, kb, vec, ln, a, E)  # noqa: E731
+    wv, wl = _bwd(lib, kb, vec, ln, (gY, gf, gc, None, None, None), E)
+    for l1, l2, add in ((None, None, z(E)), (g1, None, g1), (g1, g2, g1 + g2)):
+        gv, gl = out(gY, gf, gc, None, None, None, l1, l2)
+        assert np.array_equal(gv, wv) and np.array_equal(gl, wl + add)
+        gv, gl = out(gY, None, None, None, None, None, l1, l2)
+        assert np.array_equal(gv, wv) and np.array_equal(gl, add)
+
+
+def _bwd(lib, name, vec, ln, gs, E):
+    gv, gl = np.zeros((E, 3), np.float32), np.zeros(E, np.float32)
+    _call(getattr(lib, 'run_' + name), vec, ln, *gs[:3], gv, gl, *gs[3:], E=E)
+    return gv, gl
